@@ -8,13 +8,16 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liblelph_hip.so")
 ARCH = os.environ.get("LELPH_OFFLOAD_ARCH", "gfx950")
 
-HIP_SOURCES = ["lelph_hip.hip", "learned.hip"]
+# (source, object, extra flags); conv_inst.hip is one object per part
+HIP_SOURCES = [("lelph_hip.hip", "lelph_hip.o", []), ("learned.hip", "learned.o", [])] + [
+    ("conv_inst.hip", f"conv_inst{p}.o", [f"-DCONV_PART={p}"]) for p in range(11)]
 C_SOURCES = ["driver.c", "qeread.c", "asr.c", "phonon.c"]
 HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -53,14 +56,16 @@ def build(verbose: bool = False) -> str:
     build_nc4(verbose)
     bdir = os.path.join(HERE, "_build")
     os.makedirs(bdir, exist_ok=True)
-    objs = []
-    for src in HIP_SOURCES:
-        obj = os.path.join(bdir, os.path.splitext(src)[0] + ".o")
-        cmd = [_hipcc(), *HIPCC_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        subprocess.run(cmd, check=True)
+    objs, cmds = [], []
+    for src, name, extra in HIP_SOURCES:
+        obj = os.path.join(bdir, name)
+        cmds.append([_hipcc(), *HIPCC_FLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
+    with ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as ex:
+        for cmd, done in [(c, ex.submit(subprocess.run, c, check=True)) for c in cmds]:
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            done.result()
     for src in C_SOURCES:
         obj = os.path.join(bdir, os.path.splitext(src)[0] + ".o")
         cmd = ["gcc", "-O2", "-fPIC", "-std=c99", "-Wall", "-c", os.path.join(CSRC, src),

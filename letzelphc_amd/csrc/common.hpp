@@ -49,6 +49,17 @@ __host__ __device__ inline cpx<T> cscale(cpx<T> a, T s)
     return {a.x * s, a.y * s};
 }
 
+// per-side geometry, computed on the host in FP64 (compute_Vbare_loc.c:93-147)
+struct SideGeom
+{
+    double M[9];    // lat^T S : cartesian G (no 2pi) -> crystal, rotated
+    double G0c[3];  // crystal G shift (k+q side: lat^T (S_kq k_kq - S_k k - q))
+    double kc[3];   // crystal k of the rotated point (for the phase)
+    double tauc[3]; // fractional translation, crystal
+    int conj;       // time reversal: conjugate the coefficients
+    z64 su2[4];     // spinor rotation
+};
+
 // e^{sgn 2 pi i G0.r} at grid point p = (ix, iy, iz) (r = (ix/Nx, iy/Ny,
 // iz/Nz) in crystal units): G0.r reduced exactly in integers, the fraction
 // in FP64, rounded once to T

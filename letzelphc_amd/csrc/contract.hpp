@@ -13,47 +13,16 @@
 // The A operand dV.psi_k is formed while staging tiles into LDS, so it never
 // touches HBM.  The reduction is split over K; partials are reduced in a
 // fixed order in FP64 (no float atomics: deterministic).
-//
-// MFMA lane layouts used (16x16x4, wave64): A: lane l holds A[l%16][l/16];
-// B: lane l holds B[l/16][l%16]; D: lane l, register v holds D[row][l%16]
-// with row = Mfma<T>::row(l, v) (FP64: l/16 + 4v, measured on gfx950;
-// FP32: 4(l/16) + v).
 #pragma once
 
 #include "common.hpp"
-
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-typedef float flt4 __attribute__((ext_vector_type(4)));
-
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<double>
-{
-    typedef dbl4 acc;
-    static __device__ inline acc op(double a, double b, acc c)
-    {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    static __device__ inline int row(int lane, int v) { return (lane >> 4) + 4 * v; }
-};
-template <>
-struct Mfma<float>
-{
-    typedef flt4 acc;
-    static __device__ inline acc op(float a, float b, acc c)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    static __device__ inline int row(int lane, int v) { return 4 * (lane >> 4) + v; }
-};
+#include "mfma.hpp"
 
 #define CT_KC 16
 #define CT_LD (CT_KC + 1)
 #define CT_VB 2  // modes per block (wide tile; its tile count sets the K splits)
 #define CT_NB 32 // k bands (rows) per block
 #define CT_MB 64 // k+q bands (columns) per block
-#define CT_FLUSH 4
 
 // Block tile shapes: VB modes x NB rows x MB columns over 4 waves, wave w
 // taking mode w / NCG and column group w % NCG, each wave RB x CB blocks of

@@ -1,0 +1,430 @@
+// convpath.hpp -- host side of the sphere form (conv.hpp): buffers, launch
+// shapes and the sequence of one group of (k, k+q) pairs.  Included by
+// lelph_hip.hip after the context.
+//
+// A group of pairs goes through every step in one launch each, so a batch of
+// small cells costs a dozen launches and not a dozen per pair; the pairs of
+// a large cell go one by one, in chunks of modes whose x lines stay in the
+// last-level cache between the plane and the x step.
+#pragma once
+
+// sizes and launch shapes of a context's grid, from its spheres' radius
+struct ConvGeo
+{
+    bool f32 = false, two = false;
+    int r1[3], r2[3], xcls;
+    int words;
+    int nzk, nst, npw, ld; // bounds over the context's spheres
+    int64_t nrows;         // sets x spinors
+    PlaneShape conv, box;
+    bool square; // the planes have a kernel of their own
+    size_t sqlds;
+    size_t xlds;
+    int nsplit;
+};
+
+// bytes of line buffers (the planes' output) that a launch may fill.  More
+// than the 256 MB last-level cache on purpose: fewer, longer launches and
+// more sets per psi plane outweigh what the x step finds cached (96^3, FP64,
+// per pair: 39.7 ms with 128 MB, 35.6 with 512, 34.6 with 1000)
+static const int64_t CONV_LINE_BYTES = 512ll << 20;
+// modes of a launch that share a psi plane in L2 (4: 3 % slower in FP32, 16:
+// no gain), sets that a block takes in turn (32: the blocks of one psi plane
+// drift apart and miss, 3 %; 4: 2 % in starting blocks)
+static const int CONV_MODES = 8, CONV_SETS = 8;
+static const int64_t CONV_GROUP_BYTES = 2ll << 30;
+static const int CONV_GROUP_PAIRS = 256;
+
+// threads of the blocks over planes: as many waves as leave the fewest idle
+// rows and columns in their rounds, within `most` and 160 KB of LDS
+static bool conv_plane_shape(const ConvGeo& g, size_t item, int most, bool any, PlaneShape* s)
+{
+    const int Ny = g.r1[1] * g.r2[1];
+    s->cls = std::max(rx_class(g.r1[1], g.r2[1]), rx_class(g.r1[2], g.r2[2]));
+    double best = -1;
+    for (int nw = 4; nw <= most / 64; nw += any ? 1 : 4)
+    {
+        const PlaneLds l =
+            item == sizeof(z64)
+                ? plane_lds<double>(g.r1[1], g.r2[1], g.r1[2], g.r2[2], g.nzk, 64 * nw)
+                : plane_lds<float>(g.r1[1], g.r2[1], g.r1[2], g.r2[2], g.nzk, 64 * nw);
+        if (l.bytes > 160 * 1024) break;
+        // rounds of a wave over the rows and the columns, against the waves
+        // that a CU holds (by registers 8 in FP64 and 12 in FP32, or what
+        // the LDS allows)
+        const double rounds = 2.0 * cdiv(Ny, nw * ln_rows(g.r2[2])) +
+                              (double)cdiv(g.nzk, nw * ln_rows(g.r2[1]));
+        const int blocks = (int)std::min<size_t>(160 * 1024 / l.bytes,
+                                                 std::max(1, (item == sizeof(z64) ? 8 : 12) / nw));
+        const double score = blocks / rounds;
+        if (score > best * 1.001)
+        {
+            best = score;
+            s->nt = 64 * nw;
+            s->lds = l;
+        }
+    }
+    return best > 0;
+}
+
+// false where the sphere form does not apply: an axis length without a
+// compiled two-factor form or a plane that does not fit in LDS
+static bool conv_geo(const lelph_ctx* c, ConvGeo* g)
+{
+    const lelph_lattice& L = c->lat;
+    g->f32 = c->precision != LELPH_FP64;
+    g->two = L.nspinor == 2 && L.nmag == 4;
+    double rmax = 0;
+    int64_t npw = 0;
+    for (const DevWfc& w : c->wf)
+    {
+        rmax = std::max(rmax, w.rmax);
+        npw = std::max(npw, w.npw);
+    }
+    if (!npw || npw > 0x3fffffff) return false;
+    for (int i = 0; i < 3; ++i)
+        if (!rx_factors(L.fft_dims[i], &g->r1[i], &g->r2[i])) return false;
+    g->xcls = rx_class(g->r1[0], g->r2[0]);
+    g->words = (int)cdiv(L.fft_dims[0], 32);
+    // |G_i| spans at most 2 |a_i| max|k + G| in crystal units, whatever the
+    // rotation and the umklapp vector
+    int ext[3];
+    for (int i = 0; i < 3; ++i)
+    {
+        const double* a = L.alat_vec;
+        const double len = sqrt(a[i] * a[i] + a[3 + i] * a[3 + i] + a[6 + i] * a[6 + i]);
+        ext[i] = (int)std::min<double>((double)L.fft_dims[i], floor(2 * rmax * len + 1e-6) + 1);
+    }
+    g->npw = (int)npw;
+    g->ld = (int)(cdiv(npw, 16) * 16);
+    g->nzk = ext[2];
+    g->nst = (int)std::min<int64_t>((int64_t)ext[1] * ext[2], npw);
+    g->nrows = (int64_t)L.nspin * L.nbnds * L.nspinor;
+    if (g->nrows > 65535 || (int64_t)L.nmodes * g->nrows > 0x3fffffff) return false;
+    const size_t item = g->f32 ? sizeof(c32) : sizeof(z64);
+    const int cls = std::max(rx_class(g->r1[1], g->r2[1]), rx_class(g->r1[2], g->r2[2]));
+    const int most = g->f32 ? (g->two ? plane_threads<float, true>(cls)
+                                      : plane_threads<float, false>(cls))
+                            : (g->two ? plane_threads<double, true>(cls)
+                                      : plane_threads<double, false>(cls));
+    if (!conv_plane_shape(*g, item, most, true, &g->conv)) return false;
+    g->square = !g->two && rx_square(L.fft_dims[1], L.fft_dims[2]);
+    if (g->square)
+    {
+        const int r1 = g->r1[1], r2 = g->r2[1];
+        const int nw = g->f32 ? rx_square_waves<float>(r1 * r2) : rx_square_waves<double>(r1 * r2);
+        const int rb = g->f32 ? ln_row_bytes<float>(r1, r2) : ln_row_bytes<double>(r1, r2);
+        g->sqlds = (((size_t)nw * ln_space(r2) * rb + 15) & ~(size_t)15) +
+                   ((item * (size_t)g->nzk * ln_prow(r1, r2) + 15) & ~(size_t)15) +
+                   ((2 * (size_t)g->nzk * r1 * r2 + 15) & ~(size_t)15) +
+                   (sq_tw_lds(r1) ? sizeof(z64) * r1 * r2 : 0);
+        g->square = g->sqlds <= 160 * 1024;
+    }
+    if (!conv_plane_shape(*g, item, cls == 0 ? 512 : 256, false, &g->box)) return false;
+    g->xlds = g->f32 ? x_lds<float>(g->r1[0], g->r2[0]) : x_lds<double>(g->r1[0], g->r2[0]);
+    if (g->xlds > 160 * 1024) return false;
+    // K splits of the sphere product: enough blocks for one pair alone, at
+    // least 8 chunks each; from the shape only, so that a pair's sums do not
+    // depend on what it is batched with
+    const int64_t tiles = sph_gemm_tiles(L.nmodes, L.nbnds) * L.nspin;
+    const int64_t chunks = cdiv(npw, SG_KC) * L.nspinor;
+    g->nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(cdiv(1024, tiles), chunks / 8));
+    return true;
+}
+
+// pairs that go through the steps together, and the modes and sets of a
+// plane launch
+struct ConvGroup
+{
+    int np, nv, ns;
+};
+
+static ConvGroup conv_group(const lelph_ctx* c, const ConvGeo& g, int64_t npairs)
+{
+    const lelph_lattice& L = c->lat;
+    const int64_t item = g.f32 ? sizeof(c32) : sizeof(z64);
+    const int64_t one = item * L.fft_dims[0] * g.nst; // lines of one mode and set
+    const int64_t gsz = (int64_t)L.nmodes * L.nspin * L.nbnds * L.nbnds;
+    const int64_t pair = item * g.nrows * (c->nf + L.fft_dims[0] * (int64_t)g.nst +
+                                           (int64_t)(L.nmodes + 2) * g.ld) +
+                         (int64_t)sizeof(z64) * g.nsplit * gsz;
+    const int64_t room = std::max<int64_t>(1, CONV_LINE_BYTES / one); // (mode, set) lines
+    int64_t p = std::min<int64_t>(npairs, CONV_GROUP_PAIRS);
+    p = std::min(p, std::max<int64_t>(1, room / (L.nmodes * g.nrows)));
+    p = std::min(p, std::max<int64_t>(1, CONV_GROUP_BYTES / pair));
+    p = std::min<int64_t>(p, 65535 / std::max(1, L.nspin) / 2);
+    ConvGroup r;
+    r.np = (int)std::max<int64_t>(1, p);
+    // one pair: up to 8 modes share a psi plane, the sets fill the rest
+    int64_t nv = L.nmodes, ns = g.nrows;
+    if (nv * ns * r.np > room)
+    {
+        nv = std::min<int64_t>(L.nmodes, CONV_MODES);
+        nv = std::max<int64_t>(1, std::min(nv, room));
+        ns = std::max<int64_t>(1, std::min<int64_t>(g.nrows, room / nv));
+        if (ns == g.nrows) nv = std::max<int64_t>(1, std::min<int64_t>(L.nmodes, room / ns));
+    }
+    nv = std::max<int64_t>(1, std::min<int64_t>(nv, 500000 / ns)); // grid rows
+    r.nv = (int)nv;
+    r.ns = (int)ns;
+    return r;
+}
+
+// the FP32 potential with its rows in the plane kernels' order
+static int conv_ensure_dv32(lelph_ctx* c, const ConvGeo& g)
+{
+    if (c->cv_dv32_valid) return LELPH_OK;
+    const int64_t n = (int64_t)c->lat.nmodes * c->lat.nmag * c->nf;
+    LELPH_TRY(c->cv_dv32.ensure(sizeof(c32) * n));
+    hipLaunchKernelGGL(k_conv_dv32<float>, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, c->stream,
+                       c->dv64.as<z64>(), c->cv_dv32.as<c32>(), n, (int)c->lat.fft_dims[2],
+                       g.r1[2], g.r2[2]);
+    HIP_TRY(hipGetLastError());
+    c->cv_dv32_valid = true;
+    return LELPH_OK;
+}
+
+// local part of `np` pairs into g (device, np * gsz contiguous) on stream
+// st.  ev: [1] boxes built, [2] products done, or NULL.  desc: the group's
+// descriptors, uploaded unless they are there already (a captured pass).
+template <typename T>
+static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc, bool upload,
+                      const double* qpt, const lelph_pair* pairs, int np, const ConvGroup& gr,
+                      z64* g, hipStream_t st, hipEvent_t* ev)
+{
+    const lelph_lattice& L = c->lat;
+    const int nv = gr.nv, nset = gr.ns;
+    const int Nx = (int)L.fft_dims[0], Ny = (int)L.fft_dims[1], Nz = (int)L.fft_dims[2];
+    const int nmag_eff = (L.nspinor == 1 && L.nmag == 4) ? 1 : L.nmag;
+    // sides: every pair's k+q sphere, then the distinct k ones
+    std::vector<SphSide> sides((size_t)np);
+    std::vector<ConvPair> cp((size_t)np);
+    std::vector<int> kside((size_t)np);
+    std::vector<std::pair<int64_t, int>> keys;
+    for (int i = 0; i < np; ++i)
+    {
+        const lelph_pair& p = pairs[i];
+        if (p.ik < 0 || p.ikq < 0 || p.ik >= (int)c->wf.size() || p.ikq >= (int)c->wf.size())
+            return LELPH_ERR_ARG;
+        if (p.ksym < 0 || p.kqsym < 0 || p.ksym >= L.nsym || p.kqsym >= L.nsym)
+            return LELPH_ERR_ARG;
+        if (!c->wf[p.ik].wfc || !c->wf[p.ikq].wfc) return LELPH_ERR_STATE;
+        SideGeom gk;
+        LELPH_TRY(local_geometry(c, qpt, p.ikq, p.ik, p.kqsym, p.ksym, &sides[i].geo, &gk));
+        sides[i].wfc = c->wf[p.ikq].wfc;
+        sides[i].gvec = c->wf[p.ikq].gvec;
+        sides[i].npw = (int)c->wf[p.ikq].npw;
+        const int64_t key = (int64_t)p.ik * L.nsym + p.ksym;
+        int at = -1;
+        for (const auto& k : keys)
+            if (k.first == key) at = k.second;
+        if (at < 0)
+        {
+            at = (int)sides.size();
+            keys.push_back({key, at});
+            SphSide s{};
+            s.geo = gk;
+            s.wfc = c->wf[p.ik].wfc;
+            s.gvec = c->wf[p.ik].gvec;
+            s.npw = (int)c->wf[p.ik].npw;
+            sides.push_back(s);
+        }
+        kside[i] = at;
+    }
+    const int ns = (int)sides.size(), nk = ns - np;
+    // map arena of a side
+    const size_t cells = (size_t)Ny * Nz;
+    auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+    const size_t o_mask = 0, n_mask = up(4 * cells * geo.words);
+    const size_t o_ph = up(n_mask * (size_t)ns);
+    const size_t s_ph = up(sizeof(z64) * geo.npw), s_idx = up(4 * (size_t)geo.npw);
+    const size_t s_smap = up(4 * (size_t)geo.nzk * Ny), s_zc = up(2 * (size_t)Nz);
+    const size_t s_off = up(4 * (size_t)geo.nst), s_sm = up(4 * (size_t)geo.nst * geo.words);
+    const size_t per = s_ph + s_idx + s_smap + s_zc + s_off + s_sm + 256;
+    LELPH_TRY(b.map.ensure(o_ph + per * ns));
+    const size_t row = sizeof(cpx<T>) * (size_t)geo.nrows;
+    const size_t s_coef = row * geo.ld, s_line = row * Nx * geo.nst, s_box = row * c->nf;
+    LELPH_TRY(b.coef.ensure(s_coef * ns));
+    const size_t s_cl = sizeof(cpx<T>) * (size_t)nset * nv * Nx * geo.nst, s_c = s_coef * L.nmodes;
+    LELPH_TRY(b.line.ensure(std::max(s_line * nk, s_cl * np)));
+    LELPH_TRY(b.box.ensure(s_box * nk));
+    LELPH_TRY(b.c.ensure(s_c * np));
+    const int64_t gsz = (int64_t)L.nmodes * L.nspin * L.nbnds * L.nbnds;
+    if (geo.nsplit > 1) LELPH_TRY(b.part.ensure(sizeof(z64) * (size_t)geo.nsplit * np * gsz));
+    char* m0 = b.map.as<char>();
+    for (int i = 0; i < ns; ++i)
+    {
+        SphSide& s = sides[i];
+        s.ld = (int)(cdiv(s.npw, 16) * 16);
+        s.mask = reinterpret_cast<unsigned*>(m0 + o_mask + n_mask * i);
+        char* m = m0 + o_ph + per * i;
+        s.ph = reinterpret_cast<z64*>(m);
+        s.idx = reinterpret_cast<int*>(m += s_ph);
+        s.smap = reinterpret_cast<int*>(m += s_idx);
+        s.zc = reinterpret_cast<short*>(m += s_smap);
+        s.off = reinterpret_cast<int*>(m += s_zc);
+        s.smask = reinterpret_cast<unsigned*>(m += s_off);
+        s.cnt = reinterpret_cast<int*>(m += s_sm);
+        s.coef = b.coef.as<char>() + s_coef * i;
+        s.line = i < np ? nullptr : b.line.as<char>() + s_line * (i - np);
+        s.box = i < np ? nullptr : b.box.as<char>() + s_box * (i - np);
+    }
+    for (int i = 0; i < np; ++i)
+    {
+        cp[i].box = sides[kside[i]].box;
+        cp[i].dv = geo.f32 ? c->cv_dv32.p : c->dv64.p;
+        cp[i].side = i;
+        cp[i].line = b.line.as<char>() + s_cl * i;
+        cp[i].c = b.c.as<char>() + s_c * i;
+    }
+    const size_t n_s = up(sizeof(SphSide) * ns);
+    std::vector<char> hd(n_s + sizeof(ConvPair) * np);
+    std::memcpy(hd.data(), sides.data(), sizeof(SphSide) * ns);
+    std::memcpy(hd.data() + n_s, cp.data(), sizeof(ConvPair) * np);
+    if (upload)
+    {
+        LELPH_TRY(desc.ensure(hd.size()));
+        HIP_TRY(hipMemcpyAsync(desc.p, hd.data(), hd.size(), hipMemcpyHostToDevice, st));
+    }
+    const SphSide* ds = desc.as<SphSide>();
+    const ConvPair* dp = reinterpret_cast<const ConvPair*>(desc.as<char>() + n_s);
+    const z64 *Wx = axis_tw<double>(c->ax[0]), *Wy = axis_tw<double>(c->ax[1]),
+              *Wz = axis_tw<double>(c->ax[2]);
+
+    LELPH_TRY(zero_async(m0 + o_mask, n_mask * ns, st));
+    LELPH_TRY(conv_maps_launch(ns, geo.npw, st, ds, Nx, Ny, Nz, geo.words, geo.nzk, geo.nst,
+                               c->d_err));
+    const int64_t nsets = (int64_t)L.nspin * L.nbnds;
+    const int gper = 16;
+    LELPH_TRY(conv_gather_launch<T>(dim3((unsigned)cdiv(geo.ld, 256),
+                                         (unsigned)cdiv(nsets, gper), (unsigned)ns),
+                                    st, ds, nsets, L.nspinor, Ny, Nz, geo.words, gper));
+    // psi_k boxes
+    const unsigned tiles = (unsigned)cdiv(geo.nst, x_tile<T>());
+    BoxArgs ba{Nx, Ny, Nz, geo.words, geo.nrows, geo.nzk, geo.nst, 1};
+    ba.rows_per_block =
+        (int)std::max<int64_t>(1, std::min<int64_t>(8, geo.nrows * tiles * nk / 2048));
+    LELPH_TRY(conv_box_x_launch<T>(
+        geo.xcls, geo.xlds,
+        dim3(tiles, (unsigned)cdiv(geo.nrows, ba.rows_per_block), (unsigned)nk), st, ds + np, ba,
+        Wx));
+    const int64_t nx8 = 8 * cdiv(Nx, 8);
+    PlaneArgs pb{geo.box.lds.rows, geo.box.lds.prow, geo.r1[1], geo.r2[1]};
+    LELPH_TRY(conv_box_plane_launch<T>(geo.box, nx8 * geo.nrows * nk, st, ds + np, ba, pb, Wy,
+                                       Wz));
+    if (ev) HIP_TRY(hipEventRecord(ev[1], st));
+    // dV psi to the sphere, a chunk of modes at a time
+    PlaneArgs pc{geo.conv.lds.rows, geo.conv.lds.prow, geo.r1[1], geo.r2[1]};
+    for (int64_t vs = 0; vs < cdiv(L.nmodes, nv) * cdiv(geo.nrows, nset); ++vs)
+    {
+        // sets outside, modes inside: the psi boxes of the sets stay cached
+        const int v0 = (int)(vs % cdiv(L.nmodes, nv)) * nv;
+        ConvArgs a{};
+        a.Nx = Nx;
+        a.Ny = Ny;
+        a.Nz = Nz;
+        a.words = geo.words;
+        a.nm = L.nmodes;
+        a.v0 = v0;
+        a.nv = std::min(nv, L.nmodes - v0);
+        a.s0 = (int)(vs / cdiv(L.nmodes, nv)) * nset;
+        a.ns = (int)std::min<int64_t>(nset, geo.nrows - a.s0);
+        a.nspin = L.nspin;
+        a.nb = L.nbnds;
+        a.nspinor = L.nspinor;
+        a.nmag = nmag_eff;
+        a.nzk_max = geo.nzk;
+        a.nst_max = geo.nst;
+        const int64_t planes = (int64_t)a.ns * Nx * a.nv * np;
+        a.sper = (int)std::max<int64_t>(1, std::min<int64_t>(CONV_SETS, planes / 1024));
+        const int64_t blocks = nx8 * a.nv * cdiv(a.ns, a.sper) * np;
+        if (geo.square)
+            LELPH_TRY(conv_square_launch<T>(geo.sqlds, blocks, st, dp, ds, a, Wz));
+        else
+            LELPH_TRY(conv_plane_launch<T>(geo.two, geo.conv, blocks, st, dp, ds, a, pc, Wy, Wz));
+        const int64_t rows = (int64_t)a.ns * a.nv;
+        a.rows_per_block =
+            (int)std::max<int64_t>(1, std::min<int64_t>(8, rows * tiles * np / 4096));
+        LELPH_TRY(conv_x_launch<T>(geo.xcls, geo.xlds,
+                                   dim3(tiles, (unsigned)cdiv(rows, a.rows_per_block),
+                                        (unsigned)np),
+                                   st, dp, ds, a, Wx));
+    }
+    LELPH_TRY(sph_gemm_launch<T>(geo.nsplit, np, st, dp, ds, L.nmodes, L.nspin, L.nbnds,
+                                 L.nspinor, 1.0 / (double)c->nf,
+                                 geo.nsplit > 1 ? b.part.as<z64>() : g));
+    if (ev) HIP_TRY(hipEventRecord(ev[2], st));
+    if (geo.nsplit > 1)
+    {
+        hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(gsz * np, 256)), dim3(256), 0, st,
+                           b.part.as<z64>(), geo.nsplit, gsz * np, 1.0 / (double)c->nf, g);
+        HIP_TRY(hipGetLastError());
+    }
+    return LELPH_OK;
+}
+
+// internal status: a sphere that this form does not take (two plane waves
+// on one box point); the caller goes on in the box form
+#define LELPH_CONV_REDO 1001
+
+// Whether the local part runs in the sphere form.  Per set, mode and grid
+// point the box form costs 8 nb operations, the sphere form a transform
+// whatever nb is; measured in picoseconds (60^3 .. 96^3, 16 .. 128 bands,
+// all steps of the local part):
+//   box, FP32    0.093 per band, bands padded to 16 (57 ms per 96^3 pair of
+//                128 bands and 48 modes); FP64 0.19, with the padding of
+//                its tile; bf16x6 5.4 per tile of 128 x 64; bf16x3 on the
+//                producer/consumer kernel 2.65 at 128 bands
+//   sphere       square planes 3.3 + 0.011 nb (FP32), 5.6 (FP64), others
+//                4.5 + 0.011 nb and 6.0; a 2x2 spinor potential 5.2 and 14
+//                (box form 2.2 x)
+// Where the box form's time is a few launches, the sphere form wins by
+// taking all pairs of a group together.
+static bool conv_use(const lelph_ctx* c, ConvGeo* g)
+{
+    if (c->conv_off || !conv_geo(c, g)) return false;
+    const lelph_lattice& L = c->lat;
+    const int prec = effective_precision(c), nb = L.nbnds;
+    // a pair whose box product takes less than some 100 us
+    const double work = (double)c->nf * L.nmodes * L.nspin * L.nspinor * nb; // points x rows
+    if (work < 2e7) return true;
+    double box, sphere;
+    if (prec == LELPH_FP64)
+    {
+        const int* s = CT_SHAPES[ct_auto(L.nmodes, nb, false) - 1];
+        box = 0.19 * (double)(cdiv(L.nmodes, s[0]) * s[0]) / L.nmodes *
+              (double)(cdiv(nb, s[1]) * s[1]) / nb * (double)(cdiv(nb, s[2]) * s[2]);
+        sphere = g->two ? 14.0 : g->square ? 5.6 : 6.0;
+    }
+    else
+    {
+        sphere = (g->two ? 5.2 : g->square ? 3.3 : 4.5) + 0.011 * nb;
+        if (prec == LELPH_FP32)
+            box = 0.093 * (double)(cdiv(nb, 16) * 16) * (double)(cdiv(nb, 16) * 16) / nb;
+        else if (prec == LELPH_BF16X6)
+            box = 5.4 * (double)(cdiv(nb, 128) * 128) * (double)(cdiv(nb, 64) * 64) /
+                  (128.0 * nb);
+        else
+            box = 2.65 * (double)(cdiv(nb, 16) * 16) * (double)(cdiv(nb, 128) * 128) /
+                  (128.0 * nb);
+    }
+    if (g->two && prec != LELPH_BF16X6) box *= 2.2;
+    return sphere < box;
+}
+
+// the potential in the precision that the sphere form reads
+static int conv_prepare(lelph_ctx* c, const ConvGeo& geo)
+{
+    if (!c->dv_set) return LELPH_ERR_STATE;
+    if (c->lat.nmag == 2 && (c->lat.nspin != 2 || c->lat.nspinor != 1)) return LELPH_ERR_ARG;
+    return geo.f32 ? conv_ensure_dv32(c, geo) : LELPH_OK;
+}
+
+static int conv_group_local(lelph_ctx* c, const ConvGeo& geo, const ConvGroup& gr, ConvBufs& b,
+                            DBuf& desc, bool upload, const double* qpt, const lelph_pair* pairs,
+                            int np, z64* g, hipStream_t st, hipEvent_t* ev)
+{
+    return geo.f32
+               ? conv_local<float>(c, geo, b, desc, upload, qpt, pairs, np, gr, g, st, ev)
+               : conv_local<double>(c, geo, b, desc, upload, qpt, pairs, np, gr, g, st, ev);
+}

@@ -24,6 +24,7 @@
 #include "split.hpp"
 #include "splitpc.hpp"
 #include "boxes.hpp"
+#include "conv_launch.hpp"
 #include "dmats.hpp"
 #include "interp.hpp"
 #include "dyn.hpp"
@@ -40,6 +41,7 @@ struct DevWfc
     z64* wfc = nullptr;
     double* gvec = nullptr;
     double* Fk = nullptr;
+    double rmax = 0; // largest |k + G|, cartesian without 2pi
 };
 
 // a growable device buffer
@@ -77,6 +79,8 @@ struct DBuf
 };
 
 } // namespace
+
+#include "convpath_bufs.hpp"
 
 struct lelph_ctx
 {
@@ -141,6 +145,10 @@ struct lelph_ctx
     DBuf idx_k, idx_kq, ph_k, ph_kq, box_k, box_kq, part, g, gbatch, presplit;
     // pruned transforms: per side x-plane counts, offsets, cursors, G order
     DBuf pl_cnt[2], pl_off[2], pl_cur[2], pl_perm[2];
+    // sphere form of the local part
+    ConvBufs cv;
+    DBuf cv_dv32;
+    bool cv_dv32_valid = false;
     // electronic representation matrices
     DBuf dm_map, dm_ph, dm_pos, dm_wRS, dm_wS2, dm_part, dm_out;
     // q-star rotation
@@ -204,6 +212,7 @@ struct lelph_ctx
     // around build_boxes by the bf16 split paths); where build_boxes left
     // the k+q box and the umklapp vector its consumer applies
     bool box_defer = false;
+    bool conv_off = false; // a sphere that the sphere form does not take was met
     const void* kq_view = nullptr;
     int kq_g0[3] = {0, 0, 0};
 
@@ -806,6 +815,10 @@ static void launch_contract(int shape, bool sep, dim3 grid, hipStream_t st, cons
     }
 }
 
+static int effective_precision(const lelph_ctx* c);
+
+#include "convpath.hpp"
+
 // local part into g (device): elphLocal
 template <typename T>
 static int run_local(lelph_ctx* c, const double* qpt, const lelph_pair& pr, z64* g,
@@ -848,7 +861,6 @@ static int run_local(lelph_ctx* c, const double* qpt, const lelph_pair& pr, z64*
 // non-local part of one pair on stream st; its last kernel adds into g and
 // waits for mode_after first when that is given (the local part of the same
 // pair, which writes g, runs on the context stream)
-static int effective_precision(const lelph_ctx* c);
 
 // one side's <beta|psi> projector GEMM into out (rows, ncol) from the beta /
 // psi pieces of k_nl_presplit on BF16 MFMA (NP pieces, NPROD products),
@@ -1225,6 +1237,14 @@ static int run_local_split(lelph_ctx* c, const double* qpt, const lelph_pair& pr
 static int run_local_any(lelph_ctx* c, const double* qpt, const lelph_pair& pr, z64* g,
                          hipEvent_t* ev)
 {
+    ConvGeo geo;
+    if (conv_use(c, &geo))
+    {
+        LELPH_TRY(conv_prepare(c, geo));
+        c->box_sides = 2;
+        return conv_group_local(c, geo, conv_group(c, geo, 1), c->cv, c->cv.desc, true, qpt, &pr,
+                                1, g, c->stream, ev);
+    }
     switch (c->precision)
     {
         case LELPH_FP64: return run_local<double>(c, qpt, pr, g, ev);
@@ -1256,7 +1276,8 @@ static int check_err(lelph_ctx* c)
     int e = 0;
     LELPH_TRY(read_err(c, &e));
     if (e & 2) return LELPH_ERR_SYM;
-    if (e) return LELPH_ERR_RANGE;
+    if (e & 7) return LELPH_ERR_RANGE;
+    if (e) return LELPH_CONV_REDO;
     return LELPH_OK;
 }
 
@@ -1309,6 +1330,8 @@ static void free_ctx(lelph_ctx* c)
                     c->d_fco,   c->d_fco_off, c->d_err, c->d_gco,  c->d_vlocg, c->d_vploc};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    c->cv.release();
+    c->cv_dv32.release();
     DBuf* bufs[] = {&c->dv64, &c->dv32, &c->eig_d, &c->vloc_tmp, &c->rot_tmp, &c->idx_k,
                     &c->idx_kq, &c->ph_k, &c->ph_kq, &c->box_k, &c->box_kq, &c->box_x, &c->part, &c->g,
                     &c->gbatch, &c->presplit, &c->nlK, &c->nlKp, &c->Y_K, &c->Y_Kp, &c->wr_K, &c->wr_Kp,
@@ -1539,6 +1562,14 @@ int lelph_upload_wfc(lelph_ctx* c, int64_t ik, const double* wfc, const double* 
     w = DevWfc{};
     const int64_t nset = (int64_t)c->lat.nspin * c->lat.nbnds * c->lat.nspinor;
     w.npw = npw;
+    const double* kp = c->kpt_ibz.data() + 3 * ik;
+    for (int64_t g = 0; g < npw; ++g)
+    {
+        const double x = kp[0] + gvec[3 * g], y = kp[1] + gvec[3 * g + 1],
+                     z = kp[2] + gvec[3 * g + 2];
+        w.rmax = std::max(w.rmax, x * x + y * y + z * z);
+    }
+    w.rmax = sqrt(w.rmax);
     HIP_TRY(hipMalloc(&w.wfc, sizeof(z64) * nset * npw));
     HIP_TRY(hipMemcpy(w.wfc, wfc, sizeof(z64) * nset * npw, hipMemcpyHostToDevice));
     HIP_TRY(hipMalloc(&w.gvec, sizeof(double) * 3 * npw));
@@ -1755,7 +1786,7 @@ int lelph_set_dvscf(lelph_ctx* c, const double qpt[3], const double* eigVec, con
     const int64_t ld = (int64_t)L.nmag * c->nf;
     const size_t bytes = sizeof(z64) * (size_t)nm * ld;
     c->dv_set = false;
-    c->dv32_valid = false;
+    c->dv32_valid = c->cv_dv32_valid = false;
     LELPH_TRY(set_eig(c, eigVec));
     LELPH_TRY(c->dv64.ensure(bytes));
     const bool screened = (kernel == LELPH_KERNEL_DFPT || kernel == LELPH_KERNEL_DFPT_LOCAL);
@@ -1880,10 +1911,10 @@ static int ensure_out_ring(lelph_ctx* c, size_t slice)
     return LELPH_OK;
 }
 
-static int finish_timings(lelph_ctx* c, int64_t npairs)
+static int finish_timings(lelph_ctx* c, int64_t ngroups, int64_t npairs)
 {
     double t[5] = {0, 0, 0, 0, 0};
-    for (int64_t i = 0; i < npairs; ++i)
+    for (int64_t i = 0; i < ngroups; ++i)
     {
         hipEvent_t* e = c->evs.data() + 5 * i;
         float a = 0;
@@ -1912,14 +1943,25 @@ static int one_pair(lelph_ctx* c, const double* qpt, int ikq, int ik, int kqsym,
     const int64_t gsz = (int64_t)c->lat.nmodes * c->lat.nspin * c->lat.nbnds * c->lat.nbnds;
     LELPH_TRY(c->g.ensure(sizeof(z64) * gsz));
     LELPH_TRY(ensure_events(c, 1));
-    c->box_sides = 0;
-    if (accumulate)
-        HIP_TRY(hipMemcpyAsync(c->g.p, host_g, sizeof(z64) * gsz, hipMemcpyHostToDevice,
-                               c->stream));
-    LELPH_TRY(gkq_device(c, qpt, pr, local, nonloc, c->g.as<z64>(), c->evs.data()));
-    HIP_TRY(hipMemcpyAsync(host_g, c->g.p, sizeof(z64) * gsz, hipMemcpyDeviceToHost, c->stream));
-    LELPH_TRY(check_err(c));
-    return finish_timings(c, 1);
+    for (;;)
+    {
+        c->box_sides = 0;
+        if (accumulate)
+            HIP_TRY(hipMemcpyAsync(c->g.p, host_g, sizeof(z64) * gsz, hipMemcpyHostToDevice,
+                                   c->stream));
+        LELPH_TRY(gkq_device(c, qpt, pr, local, nonloc, c->g.as<z64>(), c->evs.data()));
+        HIP_TRY(hipMemcpyAsync(host_g, c->g.p, sizeof(z64) * gsz,
+                               hipMemcpyDeviceToHost, c->stream));
+        const int st = check_err(c);
+        if (st == LELPH_CONV_REDO)
+        {
+            c->conv_off = true;
+            continue;
+        }
+        LELPH_TRY(st);
+        break;
+    }
+    return finish_timings(c, 1, 1);
 }
 
 int lelph_elph_local(lelph_ctx* c, const double qpt[3], int ikq, int ik, int kqsym, int ksym,
@@ -1943,6 +1985,105 @@ int lelph_gkq(lelph_ctx* c, const double qpt[3], int ikq, int ik, int kqsym, int
     return one_pair(c, qpt, ikq, ik, kqsym, ksym, 1, non_loc ? 1 : 0, elph_kq, 0);
 }
 
+extern "C++" {
+// psi sides that a walk along k -> k+q chains leaves: a head's two, one per
+// linked pair, none for the k+q side that closes a cycle on its head
+static int64_t chain_sides(const lelph_pair* pairs, const std::vector<int64_t>& order)
+{
+    int64_t n = 0;
+    const lelph_pair* head = nullptr;
+    const lelph_pair* prev = nullptr;
+    for (int64_t i : order)
+    {
+        const lelph_pair& p = pairs[i];
+        const bool link = prev && prev->ikq == p.ik && prev->kqsym == p.ksym;
+        if (!link)
+        {
+            head = &p;
+            ++n;
+        }
+        const bool close = head->ik == p.ikq && head->ksym == p.kqsym;
+        if (!close) ++n;
+        prev = &p;
+    }
+    return n;
+}
+
+// lelph_gkq_batch in the sphere form: groups of pairs, their non-local parts
+// on the second stream along the chains, each group's g copied out while
+// later groups compute
+static int conv_batch(lelph_ctx* c, const ConvGeo& geo, const double* qpt, int64_t npairs,
+                      const lelph_pair* pairs, int non_loc, double* g_out)
+{
+    const int64_t gsz = (int64_t)c->lat.nmodes * c->lat.nspin * c->lat.nbnds * c->lat.nbnds;
+    std::vector<int64_t> order;
+    chain_order(c, pairs, npairs, order);
+    LELPH_TRY(conv_prepare(c, geo));
+    const ConvGroup gr = conv_group(c, geo, npairs);
+    const int np = gr.np;
+    const int64_t ngroups = cdiv(npairs, np);
+    const size_t slice = sizeof(z64) * (size_t)gsz;
+    LELPH_TRY(ensure_out_ring(c, slice * np));
+    if (!c->nl_stream) HIP_TRY(hipStreamCreateWithFlags(&c->nl_stream, hipStreamNonBlocking));
+    char* ring = static_cast<char*>(c->out_ring);
+    auto land = [&](int64_t gi) -> int {
+        const int slot = (int)(gi % LELPH_OUT_SLOTS);
+        HIP_TRY(hipEventSynchronize(c->out_ev[slot]));
+        const int64_t p0 = gi * np, p1 = std::min(npairs, p0 + np);
+        for (int64_t p = p0; p < p1; ++p)
+            std::memcpy(g_out + 2 * order[p] * gsz,
+                        ring + slot * slice * np + (p - p0) * slice, slice);
+        return LELPH_OK;
+    };
+    c->box_sides = chain_sides(pairs, order);
+    c->nl_chain = true;
+    c->nl_prev_valid = false;
+    c->nl_head_valid = false;
+    std::vector<lelph_pair> grp((size_t)np);
+    int64_t landed = 0;
+    auto body = [&](int64_t gi) -> int {
+        const int64_t p0 = gi * np, n = std::min<int64_t>(np, npairs - p0);
+        for (int64_t i = 0; i < n; ++i) grp[i] = pairs[order[p0 + i]];
+        hipEvent_t* ev = c->evs.data() + 5 * gi;
+        z64* g = c->gbatch.as<z64>() + p0 * gsz;
+        HIP_TRY(hipEventRecord(ev[0], c->stream));
+        LELPH_TRY(conv_group_local(c, geo, gr, c->cv, c->cv.desc, true, qpt, grp.data(), (int)n,
+                                   g, c->stream, ev));
+        HIP_TRY(hipEventRecord(ev[3], c->stream));
+        if (non_loc)
+        {
+            for (int64_t i = 0; i < n; ++i)
+                LELPH_TRY(run_nonlocal(c, grp[i], g + i * gsz, c->nl_stream, ev[3]));
+            HIP_TRY(hipEventRecord(ev[4], c->nl_stream));
+        }
+        else
+            HIP_TRY(hipEventRecord(ev[4], c->stream));
+        if (gi >= LELPH_OUT_SLOTS) LELPH_TRY(land(landed++));
+        const int slot = (int)(gi % LELPH_OUT_SLOTS);
+        HIP_TRY(hipStreamWaitEvent(c->out_stream, ev[4], 0));
+        HIP_TRY(hipMemcpyAsync(ring + slot * slice * np, g, slice * n, hipMemcpyDeviceToHost,
+                               c->out_stream));
+        HIP_TRY(hipEventRecord(c->out_ev[slot], c->out_stream));
+        return LELPH_OK;
+    };
+    int st = LELPH_OK;
+    for (int64_t gi = 0; gi < ngroups && st == LELPH_OK; ++gi) st = body(gi);
+    c->nl_chain = false;
+    c->nl_prev_valid = false;
+    c->nl_head_valid = false;
+    if (st != LELPH_OK)
+    {
+        (void)hipStreamSynchronize(c->nl_stream);
+        (void)hipStreamSynchronize(c->out_stream);
+        (void)hipStreamSynchronize(c->stream);
+        return st;
+    }
+    while (landed < ngroups) LELPH_TRY(land(landed++));
+    LELPH_TRY(check_err(c));
+    return finish_timings(c, ngroups, npairs);
+}
+}
+
 int lelph_gkq_batch(lelph_ctx* c, const double qpt[3], int64_t npairs, const lelph_pair* pairs,
                     int non_loc, double* g_out)
 {
@@ -1957,6 +2098,13 @@ int lelph_gkq_batch(lelph_ctx* c, const double qpt[3], int64_t npairs, const lel
             return LELPH_ERR_ARG;
         if (p.ksym < 0 || p.kqsym < 0 || p.ksym >= c->lat.nsym || p.kqsym >= c->lat.nsym)
             return LELPH_ERR_ARG;
+    }
+    ConvGeo geo;
+    if (npairs > 0 && conv_use(c, &geo))
+    {
+        const int st = conv_batch(c, geo, qpt, npairs, pairs, non_loc, g_out);
+        if (st != LELPH_CONV_REDO) return st;
+        c->conv_off = true;
     }
     // order the pairs along k -> k+q chains, so every second psi box is
     // reused (build_boxes); results keep the caller's order
@@ -2017,7 +2165,7 @@ int lelph_gkq_batch(lelph_ctx* c, const double qpt[3], int64_t npairs, const lel
     }
     while (landed < npairs) LELPH_TRY(land(landed++));
     LELPH_TRY(check_err(c));
-    return finish_timings(c, npairs);
+    return finish_timings(c, npairs, npairs);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -2059,6 +2207,18 @@ struct lelph_multi
     std::vector<MultiPair> pairs;
     std::vector<int64_t> border; // box build order: each cell's pairs along chains
     int non_loc = 1;
+    // cells in the sphere form: their buffers and, per group of pairs, the
+    // descriptors that the captured pass reads
+    struct ConvCell
+    {
+        bool on = false;
+        ConvGeo geo;
+        ConvGroup gr{1, 1, 1};
+        ConvBufs bufs;
+        std::vector<DBuf> desc;
+        std::vector<lelph_pair> pairs;
+    };
+    std::vector<ConvCell> conv;
     std::vector<DBuf> gdev;    // per cell: (npairs, nmodes, nspin, nb, nb) complex128
     std::vector<void*> ghost;  // per cell: pinned copy of gdev
     std::vector<size_t> gbytes;
@@ -2127,6 +2287,7 @@ static hipError_t launch_queue(int prec, bool sep, int shape, int grid, hipStrea
 // issues the whole batch on m->stream (eagerly with events, or under capture)
 static int multi_enqueue(lelph_multi* m, bool timed)
 {
+    const bool first = timed; // the eager pass also uploads the descriptors
     struct Saved
     {
         hipStream_t st;
@@ -2185,6 +2346,7 @@ static int multi_enqueue(lelph_multi* m, bool timed)
         for (int64_t bi : m->border)
         {
             MultiPair& p = m->pairs[(size_t)bi];
+            if (m->conv[p.cell].on) continue;
             lelph_ctx* c = m->ctx[p.cell];
             c->box_k.p = p.kbox;
             c->box_k.n = p.bb;
@@ -2200,6 +2362,22 @@ static int multi_enqueue(lelph_multi* m, bool timed)
                 LELPH_TRY(build_boxes<float>(c, q, p.pr, kf, kg, nullptr, kqf));
         }
         if (timed) HIP_TRY(hipEventRecord(m->ev[1], m->stream));
+        // cells in the sphere form, group by group straight into their g
+        for (size_t i = 0; i < m->ctx.size(); ++i)
+        {
+            auto& cc = m->conv[i];
+            lelph_ctx* c = m->ctx[i];
+            const int64_t gsz =
+                (int64_t)c->lat.nmodes * c->lat.nspin * c->lat.nbnds * c->lat.nbnds;
+            for (size_t k = 0; cc.on && k < cc.desc.size(); ++k)
+            {
+                const int64_t p0 = (int64_t)k * cc.gr.np;
+                const int n = (int)std::min<int64_t>(cc.gr.np, (int64_t)cc.pairs.size() - p0);
+                LELPH_TRY(conv_group_local(c, cc.geo, cc.gr, cc.bufs, cc.desc[k], first,
+                                           m->qpt[i].data(), cc.pairs.data() + p0, n,
+                                           m->gdev[i].as<z64>() + p0 * gsz, m->stream, nullptr));
+            }
+        }
         // the work-queue contractions
         LELPH_TRY(zero_async(m->counter.p, sizeof(int) * m->queues.size(), m->stream));
         for (size_t qi = 0; qi < m->queues.size(); ++qi)
@@ -2215,6 +2393,7 @@ static int multi_enqueue(lelph_multi* m, bool timed)
         // stream, after the reductions), joined, then the copy-out
         for (auto& p : m->pairs)
         {
+            if (m->conv[p.cell].on) continue;
             lelph_ctx* c = m->ctx[p.cell];
             z64* g = m->gdev[p.cell].as<z64>() + p.index * p.gsz;
             hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(p.gsz, 256)), dim3(256), 0,
@@ -2272,7 +2451,7 @@ static int build_queue(lelph_multi* m, int prec, int shape, DBuf& qp, DBuf& qi, 
     *any_sep = false;
     for (auto& p : m->pairs)
     {
-        if (p.prec != prec || p.shape != shape) continue;
+        if (p.prec != prec || p.shape != shape || m->conv[p.cell].on) continue;
         lelph_ctx* c = m->ctx[p.cell];
         const lelph_lattice& L = c->lat;
         const int nmag_eff = (L.nspinor == 1 && L.nmag == 4) ? 1 : L.nmag;
@@ -2332,6 +2511,11 @@ static void multi_free(lelph_multi* m)
         p.part.release();
         p.ebuf.release();
     }
+    for (auto& cc : m->conv)
+    {
+        cc.bufs.release();
+        for (auto& d : cc.desc) d.release();
+    }
     for (auto& g : m->gdev) g.release();
     for (void* h : m->ghost)
         if (h) (void)hipHostFree(h);
@@ -2353,9 +2537,9 @@ static void multi_free(lelph_multi* m)
 
 extern "C" {
 
-int lelph_multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
-                       const int64_t* npairs, const lelph_pair* const* pairs, int non_loc,
-                       lelph_multi** out)
+static int multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
+                        const int64_t* npairs, const lelph_pair* const* pairs, int non_loc,
+                        lelph_multi** out)
 {
     if (!out || ncells < 1 || !ctxs || !qpts || !npairs || !pairs) return LELPH_ERR_ARG;
     *out = nullptr;
@@ -2403,7 +2587,18 @@ int lelph_multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
         m->qpt.push_back({qpts[3 * i], qpts[3 * i + 1], qpts[3 * i + 2]});
         m->npairs.push_back(npairs[i]);
         const int prec = effective_precision(c);
-        if (prec == LELPH_FP32)
+        m->conv.emplace_back();
+        auto& cc = m->conv.back();
+        cc.on = npairs[i] > 0 && conv_use(c, &cc.geo);
+        if (cc.on)
+        {
+            cc.gr = conv_group(c, cc.geo, npairs[i]);
+            cc.pairs.assign(pairs[i], pairs[i] + npairs[i]);
+            cc.desc.resize((size_t)cdiv(npairs[i], cc.gr.np));
+            int st = conv_prepare(c, cc.geo);
+            if (st != LELPH_OK) return fail(st);
+        }
+        else if (prec == LELPH_FP32)
         {
             int st = ensure_dv32(c);
             if (st != LELPH_OK) return fail(st);
@@ -2441,7 +2636,8 @@ int lelph_multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
                 return fail(gs);
             }
             for (int d = 0; d < 3; ++d) p.g0[d] = (int)std::lrint(gkq.G0c[d]);
-            if (p.box_kq.ensure(bb) || p.part.ensure(sizeof(z64) * (size_t)(p.nsplit * gsz)) ||
+            if ((!cc.on && (p.box_kq.ensure(bb) ||
+                            p.part.ensure(sizeof(z64) * (size_t)(p.nsplit * gsz)))) ||
                 (non_loc && p.ebuf.ensure(sizeof(z64) * (size_t)(3 * L.natom * es))))
             {
                 m->pairs.push_back(p);
@@ -2467,6 +2663,7 @@ int lelph_multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
                     if (p.pr.ik == q.pr.ikq && p.pr.ksym == q.pr.kqsym)
                         p.link = first + order[n - 1];
                 }
+                if (cc.on) continue;
                 const MultiPair* lp = p.link >= 0 ? &m->pairs[(size_t)p.link] : nullptr;
                 if (lp && !lp->g0[0] && !lp->g0[1] && !lp->g0[2])
                     p.kbox = lp->box_kq.p;
@@ -2524,6 +2721,7 @@ int lelph_multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
     for (lelph_ctx* c : m->ctx)
     {
         st = check_err(c);
+        if (st == LELPH_CONV_REDO) c->conv_off = true;
         if (st != LELPH_OK) return fail(st);
     }
     if (hipStreamBeginCapture(m->stream, hipStreamCaptureModeRelaxed) != hipSuccess)
@@ -2541,6 +2739,18 @@ int lelph_multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
     }
     *out = m;
     return LELPH_OK;
+}
+
+int lelph_multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
+                       const int64_t* npairs, const lelph_pair* const* pairs, int non_loc,
+                       lelph_multi** out)
+{
+    // again where a cell turned out not to fit the sphere form (each such
+    // cell is in the box form from then on)
+    int st = LELPH_CONV_REDO;
+    for (int i = 0; i <= ncells && st == LELPH_CONV_REDO; ++i)
+        st = multi_create(ncells, ctxs, qpts, npairs, pairs, non_loc, out);
+    return st == LELPH_CONV_REDO ? LELPH_ERR_RANGE : st;
 }
 
 int lelph_multi_run(lelph_multi* m, double* const* g_out)
@@ -3278,7 +3488,7 @@ int lelph_interp_set_dvscf(lelph_ctx* c, const double qpt[3], const double* eigV
     const int64_t ld = (int64_t)L.nmag * c->nf;
     const size_t bytes = sizeof(z64) * (size_t)nm * ld;
     c->dv_set = false;
-    c->dv32_valid = false;
+    c->dv32_valid = c->cv_dv32_valid = false;
     LELPH_TRY(set_eig(c, eigVec));
     LELPH_TRY(c->dv64.ensure(bytes));
     if (kernel == LELPH_KERNEL_DFPT || kernel == LELPH_KERNEL_DFPT_LOCAL)
@@ -3404,7 +3614,7 @@ int lelph_set_dvscf_file(lelph_ctx* c, const double qpt[3], const double* eigVec
     const int64_t ld = (int64_t)L.nmag * c->nf;
     const size_t bytes = sizeof(z64) * (size_t)nm * ld;
     c->dv_set = false;
-    c->dv32_valid = false;
+    c->dv32_valid = c->cv_dv32_valid = false;
     LELPH_TRY(set_eig(c, eigVec));
     LELPH_TRY(c->dv64.ensure(bytes));
     LELPH_TRY(c->ip_tmp.ensure(bytes));

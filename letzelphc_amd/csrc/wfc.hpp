@@ -12,17 +12,6 @@
 
 #include "common.hpp"
 
-// per-side geometry, computed on the host in FP64 (compute_Vbare_loc.c:93-147)
-struct SideGeom
-{
-    double M[9];    // lat^T S : cartesian G (no 2pi) -> crystal, rotated
-    double G0c[3];  // crystal G shift (k+q side: lat^T (S_kq k_kq - S_k k - q))
-    double kc[3];   // crystal k of the rotated point (for the phase)
-    double tauc[3]; // fractional translation, crystal
-    int conj;       // time reversal: conjugate the coefficients
-    z64 su2[4];     // spinor rotation
-};
-
 // integer rotated G -> box index and translation phase.  Out-of-box G set
 // bit 1 of *err (planner.c:128-137: "gvec > Nfft dim").
 __global__ void k_gindex(const double* __restrict__ gvec, int64_t npw, SideGeom geo,

@@ -1,0 +1,89 @@
+"""The sphere form of the local part (transforms of dV psi to the k+q sphere,
+csrc/conv.hpp) against the FP64 oracle at the sizes where its layouts can go
+wrong: odd and unequal axes, lines of every factor class (products of 2, 3, 5
+and 7; both factors small, one of 15 to 18), planes with a kernel of their own
+and planes without, row counts that leave a wave's last rows idle, spheres
+that fill most of the box, rotated and time-reversed sides with an umklapp
+vector, both spins, spinors with and without the 2x2 potential.  Lengths
+without a two-factor form (11, 13, 22) run in the box form and must agree
+just as well.
+
+Bars: the FP64 form differs from the oracle by rounding of the same sums
+(1e-10, as everywhere); FP32 transforms of N points carry some
+log2(N) * 6e-8 per coefficient, averaged over the sphere (1e-6)."""
+import numpy as np
+import pytest
+
+from letzelphc_amd import lelph, synth
+from oracle import oracle as O
+
+from .util import rel_err, say
+
+pytestmark = pytest.mark.gpu
+
+GRIDS = [
+    (12, 12, 12), (15, 16, 18), (16, 15, 15), (14, 21, 20), (25, 12, 27), (28, 18, 24),
+    (12, 30, 30), (32, 14, 35), (12, 42, 16), (18, 45, 45), (12, 12, 54), (12, 56, 56),
+    (63, 12, 12), (12, 14, 70), (12, 75, 12), (12, 81, 14), (12, 96, 96), (12, 14, 108),
+    (12, 126, 12), (12, 12, 135), (144, 12, 14), (12, 160, 12), (12, 14, 216), (225, 12, 12),
+    (12, 12, 240), (13, 12, 12), (12, 22, 12), (12, 12, 26),
+]
+
+
+@pytest.mark.parametrize("fft", GRIDS)
+def test_grids(fft):
+    # the cubic cell stretched so that every axis holds the sphere
+    s = synth.tiny(nbnds=5, fft=fft, kgrid=(2, 2, 2), syms="cubic" if fft[0] == fft[1] else "id",
+                   ecut=5.0)
+    o = O.OracleSystem(s)
+    dv = o.dv_total(0)
+    pairs = synth.kq_pairs(s, 0)
+    pick = [pairs[i] for i in (0, 3, len(pairs) - 1)]
+    ref = np.stack([o.add_nonlocal(0, *p, o.elph_local(0, *p, dv)) for p in pick])
+    errs = {}
+    ctx = lelph.Context(s, "fp64")
+    try:
+        ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
+        for prec in ("fp64", "fp32"):
+            ctx.set_precision(prec)
+            errs[prec] = rel_err(ctx.gkq_batch(pick, qpt=s.qpts[0]), ref)
+    finally:
+        ctx.close()
+    say(f"case: sphere form {fft}: {errs}")
+    assert errs["fp64"] < 1e-10 and errs["fp32"] < 1e-6
+
+
+SPIN = {
+    "spin2": dict(nspin=2, nmag=2),
+    "spinor_nmag1": dict(nspinor=2, nmag=1),
+    "spinor_nmag4": dict(nspinor=2, nmag=4),
+}
+
+
+@pytest.mark.parametrize("case", list(SPIN))
+@pytest.mark.parametrize("nb", [1, 17, 33, 49])
+@pytest.mark.parametrize("fft", [(16, 16, 16), (16, 15, 18)])
+def test_bands_and_spin(case, nb, fft):
+    """column tiles of the sphere product (16, 32, 48, 64) and their
+    remainders, with the spin layouts"""
+    s = synth.tiny(nbnds=nb, fft=fft, ecut=14.0, kgrid=(2, 2, 1), syms="id", q=(0.5, 0.0, 0.0),
+                   **SPIN[case])
+    o = O.OracleSystem(s)
+    dv = o.dv_total(0)
+    pairs = synth.kq_pairs(s, 0)
+    ref = np.stack([o.elph_local(0, *p, dv) for p in pairs[:2]])
+    errs = {}
+    ctx = lelph.Context(s, "fp64")
+    try:
+        ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
+        for prec in ("fp64", "fp32"):
+            ctx.set_precision(prec)
+            one = np.stack([ctx.elph_local(*p) for p in pairs[:2]])
+            bat = ctx.gkq_batch(pairs, non_loc=False, qpt=s.qpts[0])[:2]
+            # a pair's sums do not depend on what it is batched with
+            assert np.array_equal(one, bat)
+            errs[prec] = rel_err(one, ref)
+    finally:
+        ctx.close()
+    say(f"case: sphere form {case} nb {nb} {fft}: {errs}")
+    assert errs["fp64"] < 1e-10 and errs["fp32"] < 1e-6
