@@ -112,3 +112,28 @@ __device__ inline void lds_barrier()
     } while (0)
 
 static inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Global-memory views of pointers that come out of descriptors: the compiler
+// knows the address space of kernel arguments only and would take flat
+// instructions for these, which count as LDS accesses too, so that every LDS
+// wait would also wait for the loads in flight.
+#define GLOBAL_AS __attribute__((address_space(1)))
+template <typename X>
+__device__ __forceinline__ GLOBAL_AS X* g_of(X* p)
+{
+    return (GLOBAL_AS X*)p;
+}
+template <typename T>
+struct gptr
+{
+    typedef T v2 __attribute__((ext_vector_type(2)));
+    GLOBAL_AS v2* p;
+    static __device__ __forceinline__ gptr of(const void* q) { return {(GLOBAL_AS v2*)q}; }
+    __device__ __forceinline__ cpx<T> operator[](int64_t i) const
+    {
+        const v2 x = p[i];
+        return {x.x, x.y};
+    }
+    __device__ __forceinline__ void set(int64_t i, cpx<T> v) const { p[i] = v2{v.x, v.y}; }
+    __device__ __forceinline__ gptr operator+(int64_t i) const { return {p + i}; }
+};

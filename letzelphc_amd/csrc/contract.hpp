@@ -461,34 +461,58 @@ __global__ void k_zero_words(unsigned* __restrict__ p, int64_t n)
         p[i] = 0u;
 }
 
-// g[i] = scale * sum_s part[s][i], fixed order.
-__global__ void k_reduce_parts(const z64* __restrict__ part, int nsplit, int64_t count,
-                               double scale, z64* __restrict__ g)
+// g[i] = scale * sum_s part[s][i], in an order fixed by nsplit.  Block: 32
+// elements, 8 threads each: thread u sums the parts u, u + 8, ... (four loads
+// in flight), and the eight sums are added in order.  One thread per element
+// left a chip of idle CUs waiting on a chain of loads wherever the parts are
+// many and the elements few (D matrices of 40 bands: 31 -> 9 us).
+#define RP_ELEMS 32
+template <typename P, typename G>
+__device__ __forceinline__ void reduce_body(P part, int nsplit, int64_t count, double scale, G g)
 {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
+    __shared__ double sr[8][RP_ELEMS], si[8][RP_ELEMS];
+    const int e = threadIdx.x % RP_ELEMS, u = threadIdx.x / RP_ELEMS;
+    const int64_t i = (int64_t)blockIdx.x * RP_ELEMS + e;
     double re = 0, im = 0;
-    // eight loads in flight, then their adds in split order (the same sum)
-    int s = 0;
-    for (; s + 8 <= nsplit; s += 8)
+    if (i < count)
     {
-        z64 p[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) p[u] = part[(int64_t)(s + u) * count + i];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
+        int s = u;
+        for (; s + 24 < nsplit; s += 32)
         {
-            re += p[u].x;
-            im += p[u].y;
+            z64 p[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) p[v] = part[(int64_t)(s + 8 * v) * count + i];
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+            {
+                re += p[v].x;
+                im += p[v].y;
+            }
+        }
+        for (; s < nsplit; s += 8)
+        {
+            const z64 p = part[(int64_t)s * count + i];
+            re += p.x;
+            im += p.y;
         }
     }
-    for (; s < nsplit; ++s)
+    sr[u][e] = re;
+    si[u][e] = im;
+    __syncthreads();
+    if (u != 0 || i >= count) return;
+#pragma unroll
+    for (int v = 1; v < 8; ++v)
     {
-        const z64 p = part[(int64_t)s * count + i];
-        re += p.x;
-        im += p.y;
+        re += sr[v][e];
+        im += si[v][e];
     }
-    g[i] = {re * scale, im * scale};
+    g.set(i, {scale * re, scale * im});
+}
+__global__ __launch_bounds__(256) void k_reduce_parts(const z64* __restrict__ part, int nsplit,
+                                                      int64_t count, double scale,
+                                                      z64* __restrict__ g)
+{
+    reduce_body(part, nsplit, count, scale, gptr<double>::of(g));
 }
 
 // dst[i] = (float) src[i]

@@ -356,9 +356,7 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
     if (ev) HIP_TRY(hipEventRecord(ev[2], st));
     if (geo.nsplit > 1)
     {
-        hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(gsz * np, 256)), dim3(256), 0, st,
-                           b.part.as<z64>(), geo.nsplit, gsz * np, 1.0 / (double)c->nf, g);
-        HIP_TRY(hipGetLastError());
+        LELPH_TRY(reduce_parts(b.part.as<z64>(), geo.nsplit, gsz * np, 1.0 / (double)c->nf, g, st));
     }
     return LELPH_OK;
 }

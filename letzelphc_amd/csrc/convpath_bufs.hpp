@@ -1,4 +1,5 @@
-// convpath_bufs.hpp -- device buffers of the sphere form (convpath.hpp).
+// convpath_bufs.hpp -- device buffers of the sphere form (convpath.hpp) and of
+// the non-local part (nlpath.hpp).
 // Included by lelph_hip.hip before the context, which owns a set.
 #pragma once
 
@@ -9,5 +10,40 @@ struct ConvBufs
     void release()
     {
         for (DBuf* b : {&desc, &map, &coef, &line, &box, &c, &part}) b->release();
+    }
+};
+
+// non-local part: scratch of the sides formed together, their projections,
+// the K/K' sums of a group of pairs, bf16 pieces (nl_form 1)
+struct NlBufs
+{
+    DBuf desc, side, bb, ebuf, splitA, splitB;
+    const int* kk = nullptr; // pairs' key numbers of the current window
+    void release()
+    {
+        for (DBuf* b : {&desc, &side, &bb, &ebuf, &splitA, &splitB}) b->release();
+    }
+};
+
+// the sides and pairs of one window: keys in order of first use, two key
+// numbers (k+q, k) per pair
+struct NlWindow
+{
+    std::vector<std::array<int, 2>> keys; // (iBZ k, symmetry)
+    std::vector<int> kk;
+    void add(const lelph_pair& p)
+    {
+        kk.push_back(key(p.ikq, p.kqsym));
+        kk.push_back(key(p.ik, p.ksym));
+    }
+
+  private:
+    std::map<std::array<int, 2>, int> at;
+    int key(int ik, int sym)
+    {
+        const std::array<int, 2> k = {ik, sym};
+        const auto r = at.insert({k, (int)keys.size()});
+        if (r.second) keys.push_back(k);
+        return r.first->second;
     }
 };

@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <array>
+#include <map>
 #include <mutex>
 #include <vector>
 
@@ -21,6 +22,7 @@
 #include "dvloc.hpp"
 #include "fft.hpp"
 #include "nonloc.hpp"
+#include "nlbatch.hpp"
 #include "split.hpp"
 #include "splitpc.hpp"
 #include "boxes.hpp"
@@ -179,21 +181,9 @@ struct lelph_ctx
     // device time of the last lelph_interp_dvscf: weights, R -> q, long range, total, nq
     hipEvent_t ip_ev[4] = {nullptr, nullptr, nullptr, nullptr};
     double ip_ms[5] = {0, 0, 0, 0, 0};
-    DBuf nlK, nlKp, Y_K, Y_Kp, wr_K, wr_Kp, beta_K, beta_Kp, bb_K, bb_Kp, bbpart, ebuf;
-    // non-local part along a batch's chains: <beta_K|psi> of the previous
-    // pair (key: its iBZ k+q and symmetry) serves as this pair's K' side
-    DBuf bb_Kprev;
-    bool nl_chain = false; // set while a batch issues its pairs along chains
-    bool nl_prev_valid = false;
-    int nl_prev_ik = -1, nl_prev_sym = -1;
-    // <beta_K'|psi> of the chain's head (key: its iBZ k and symmetry): the
-    // K side of a closed cycle's last pair
-    DBuf bb_Khead;
-    bool nl_head_valid = false;
-    int nl_head_ik = -1, nl_head_sym = -1;
-    // reduced-precision projector operands: FP32 copies, or bf16 piece planes
-    DBuf beta32_K, beta32_Kp, wr32_K, wr32_Kp, nlsplitA, nlsplitB;
-
+    NlBufs nl; // non-local part
+    std::vector<NlWindow> nl_win; // of the batch under way
+    int64_t nl_step = 1;          // pairs of one window
     // psi box reuse along a batch: the k+q box of the previous pair is the k
     // box of the next when their (iBZ k, symmetry) agree, up to the umklapp
     // shift of the previous k+q side
@@ -817,6 +807,17 @@ static void launch_contract(int shape, bool sep, dim3 grid, hipStream_t st, cons
 
 static int effective_precision(const lelph_ctx* c);
 
+// g = scale * the sum of nsplit partials (k_reduce_parts)
+static int reduce_parts(const z64* part, int nsplit, int64_t count, double scale, z64* g,
+                        hipStream_t st)
+{
+    hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(count, RP_ELEMS)), dim3(256), 0, st,
+                       part, nsplit, count, scale, g);
+    HIP_TRY(hipGetLastError());
+    return LELPH_OK;
+}
+
+#include "nlpath.hpp"
 #include "convpath.hpp"
 
 // local part into g (device): elphLocal
@@ -851,277 +852,7 @@ static int run_local(lelph_ctx* c, const double* qpt, const lelph_pair& pr, z64*
                        c->part.as<z64>(), nm, nb, nspin, L.nspinor, nmag_eff, c->nf, cps);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(ev[2], c->stream));
-    hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(gsz, 256)), dim3(256), 0, c->stream,
-                       c->part.as<z64>(), nsplit, gsz, 1.0 / (double)c->nf, g);
-    HIP_TRY(hipGetLastError());
-    return LELPH_OK;
-}
-
-// non-local part added onto g (device): add_elphNonLocal
-// non-local part of one pair on stream st; its last kernel adds into g and
-// waits for mode_after first when that is given (the local part of the same
-// pair, which writes g, runs on the context stream)
-
-// one side's <beta|psi> projector GEMM into out (rows, ncol) from the beta /
-// psi pieces of k_nl_presplit on BF16 MFMA (NP pieces, NPROD products),
-// FP64 split-K partials and a fixed-order FP64 reduction
-template <int NP, int NPROD>
-static int nl_gemm_split(lelph_ctx* c, const z64* A, const z64* B, int rows, int64_t ncol,
-                         int64_t npw, int conjB, z64* out, hipStream_t st)
-{
-    const int Mp = (int)(cdiv(rows, 64) * 64), Np = (int)(cdiv(ncol, 64) * 64);
-    const int64_t Kp = cdiv(npw, 32) * 32;
-    LELPH_TRY(c->nlsplitA.ensure(sizeof(__bf16) * (size_t)NP * 2 * Mp * Kp));
-    LELPH_TRY(c->nlsplitB.ensure(sizeof(__bf16) * (size_t)NP * 2 * Np * Kp));
-    hipLaunchKernelGGL((k_nl_presplit<NP>), dim3((unsigned)cdiv(Kp, 256), (unsigned)Mp), dim3(256),
-                       0, st, A, rows, npw, Mp, Kp, 0, c->nlsplitA.as<__bf16>());
-    hipLaunchKernelGGL((k_nl_presplit<NP>), dim3((unsigned)cdiv(Kp, 256), (unsigned)Np), dim3(256),
-                       0, st, B, (int)ncol, npw, Np, Kp, conjB, c->nlsplitB.as<__bf16>());
-    HIP_TRY(hipGetLastError());
-    const int64_t nchunks = Kp / 32;
-    const int64_t tiles = (int64_t)(Mp / 64) * (Np / 64);
-    int64_t cps;
-    int nsplit;
-    pick_splits(tiles, nchunks, (int64_t)rows * ncol, &cps, &nsplit);
-    const size_t need = sizeof(z64) * (size_t)nsplit * rows * ncol;
-    if (need > c->bbpart.n && st != c->stream) HIP_TRY(hipStreamSynchronize(st));
-    LELPH_TRY(c->bbpart.ensure(need));
-    hipLaunchKernelGGL((k_zgemm_nt_bf<NP, NPROD>), dim3((unsigned)tiles, (unsigned)nsplit),
-                       dim3(256), 0, st, c->nlsplitA.as<__bf16>(), c->nlsplitB.as<__bf16>(), rows,
-                       (int)ncol, Mp, Np, Kp, cps, c->bbpart.as<z64>());
-    hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv((int64_t)rows * ncol, 256)), dim3(256),
-                       0, st, c->bbpart.as<z64>(), nsplit, (int64_t)rows * ncol, 1.0, out);
-    HIP_TRY(hipGetLastError());
-    return LELPH_OK;
-}
-
-// the cart -> mode rotation of the non-local part, accumulated into g
-// (src/nonloc/Vbare_nloc.c:541-558): g += -2 pi i e^2 eig ebuf
-static int nl_mode(lelph_ctx* c, const z64* ebuf, z64* g, hipStream_t st)
-{
-    const lelph_lattice& L = c->lat;
-    const int64_t es = (int64_t)L.nspin * L.nbnds * L.nbnds;
-    const z64 pre = {0.0, -2 * LELPH_RPI * LELPH_E2};
-    hipLaunchKernelGGL(k_nl_mode, dim3((unsigned)cdiv((int64_t)L.nmodes * es, 256)), dim3(256), 0,
-                       st, ebuf, c->eig_d.as<z64>(), L.nmodes, 3 * L.natom, es, pre, g);
-    HIP_TRY(hipGetLastError());
-    return LELPH_OK;
-}
-
-// add_elphNonLocal into g on stream st; the final mode rotation waits for
-// mode_after when given.  With ebuf_out the per-atom K/K' sums go there and
-// the rotation is left to the caller (nl_mode), so g is not touched.
-static int run_nonlocal(lelph_ctx* c, const lelph_pair& pr, z64* g, hipStream_t st,
-                        hipEvent_t mode_after, z64* ebuf_out = nullptr)
-{
-    const lelph_lattice& L = c->lat;
-    if (!c->dv_set) return LELPH_ERR_STATE;
-    const DevWfc& wK = c->wf[pr.ikq];
-    const DevWfc& wKp = c->wf[pr.ik];
-    if (!wK.Fk || !wKp.Fk) return LELPH_ERR_STATE;
-    const int nlm = (c->lmax + 1) * (c->lmax + 1);
-    const int64_t nsb = (int64_t)L.nspin * L.nbnds;
-    const int64_t ncol = nsb * L.nspinor;
-    const int natom = L.natom;
-    const int rows = natom * c->pmax * 4;
-    const int64_t npm = c->npw_max;
-    LELPH_TRY(c->nlK.ensure(sizeof(double) * 3 * npm));
-    LELPH_TRY(c->nlKp.ensure(sizeof(double) * 3 * npm));
-    LELPH_TRY(c->Y_K.ensure(sizeof(double) * nlm * npm));
-    LELPH_TRY(c->Y_Kp.ensure(sizeof(double) * nlm * npm));
-    LELPH_TRY(c->wr_K.ensure(sizeof(z64) * ncol * npm));
-    LELPH_TRY(c->wr_Kp.ensure(sizeof(z64) * ncol * npm));
-    LELPH_TRY(c->beta_K.ensure(sizeof(z64) * (size_t)rows * npm));
-    LELPH_TRY(c->beta_Kp.ensure(sizeof(z64) * (size_t)rows * npm));
-    LELPH_TRY(c->bb_K.ensure(sizeof(z64) * (size_t)rows * ncol));
-    LELPH_TRY(c->bb_Kp.ensure(sizeof(z64) * (size_t)rows * ncol));
-    const int64_t es = (int64_t)L.nspin * L.nbnds * L.nbnds;
-    LELPH_TRY(c->ebuf.ensure(sizeof(z64) * (size_t)(3 * natom * es)));
-    // in a batch, the K' side of a pair whose k side is the previous pair's
-    // k+q side comes from that pair's K-side projections (k_nl_mirror)
-    const bool mirror = c->nl_chain && c->nl_prev_valid && c->nl_prev_ik == pr.ik &&
-                        c->nl_prev_sym == pr.ksym;
-    // and the K side of a pair whose k+q side is the k side of the chain's
-    // head (a closed cycle) from the head's K' projections
-    const bool close_k = c->nl_chain && c->nl_head_valid && c->nl_head_ik == pr.ikq &&
-                         c->nl_head_sym == pr.kqsym;
-    c->nl_prev_valid = false;
-    auto skip_side = [&](int side) { return side == 0 ? close_k : mirror; };
-
-    const lelph_symmetry& SK = c->syms[pr.kqsym];
-    const lelph_symmetry& SKp = c->syms[pr.ksym];
-    NlSide sK{}, sKp{};
-    std::memcpy(sK.S, SK.Rmat, sizeof(sK.S));
-    std::memcpy(sKp.S, SKp.Rmat, sizeof(sKp.S));
-    std::memcpy(sK.k, c->kpt_ibz.data() + 3 * pr.ikq, sizeof(sK.k));
-    std::memcpy(sKp.k, c->kpt_ibz.data() + 3 * pr.ik, sizeof(sKp.k));
-    std::memcpy(sK.tau, SK.tau, sizeof(sK.tau));
-    std::memcpy(sKp.tau, SKp.tau, sizeof(sKp.tau));
-    sK.conj_w = SK.time_rev ? 0 : 1;   // 'C' unless time reversed (Vbare_nloc.c:397-407)
-    sKp.conj_w = SKp.time_rev ? 1 : 0; // 'T' unless time reversed
-    LELPH_TRY(su2mat(SK.Rmat, L.nspinor, SK.time_rev, sK.su2));
-    LELPH_TRY(su2mat(SKp.Rmat, L.nspinor, SKp.time_rev, sKp.su2));
-
-    // projector GEMMs in FP32 (FP32 contexts; bf16 ones unless nl_form 1):
-    // the rotated psi is written in FP32 and beta built in FP32 only
-    const int prec = effective_precision(c);
-    const bool nl32 = prec != LELPH_FP64 &&
-                      !((prec == LELPH_BF16X3 || prec == LELPH_BF16X6) && c->tune.nl_form == 1);
-    // K, Y_lm and the rotated psi of both sides; the rotation in groups of
-    // NL_SPY sets per block row
-    constexpr int NL_SPY = 16;
-    const unsigned gy = (unsigned)std::max<int64_t>(1, cdiv(nsb, NL_SPY));
-    for (int side = 0; side < 2; ++side)
-    {
-        if (skip_side(side)) continue;
-        const DevWfc& w = side == 0 ? wK : wKp;
-        const NlSide& sd = side == 0 ? sK : sKp;
-        double* kc = side == 0 ? c->nlK.as<double>() : c->nlKp.as<double>();
-        double* y = side == 0 ? c->Y_K.as<double>() : c->Y_Kp.as<double>();
-        if (nl32)
-        {
-            DBuf& w32 = side == 0 ? c->wr32_K : c->wr32_Kp;
-            LELPH_TRY(w32.ensure(sizeof(c32) * (size_t)ncol * npm));
-            hipLaunchKernelGGL(k_nl_geom<float>, dim3((unsigned)cdiv(w.npw, 128), gy), dim3(128),
-                               0, st, w.gvec, w.npw, sd, c->lmax, w.wfc, nsb, L.nspinor, kc, y,
-                               w32.as<c32>(), NL_SPY);
-        }
-        else
-            hipLaunchKernelGGL(k_nl_geom<double>, dim3((unsigned)cdiv(w.npw, 128), gy),
-                               dim3(128), 0, st, w.gvec, w.npw, sd, c->lmax, w.wfc, nsb,
-                               L.nspinor, kc, y,
-                               side == 0 ? c->wr_K.as<z64>() : c->wr_Kp.as<z64>(), NL_SPY);
-    }
-    NlProj pj{natom, c->pmax, c->ntype};
-    if (!nl32)
-    {
-        if (!close_k)
-            hipLaunchKernelGGL(k_nl_beta<double>,
-                               dim3((unsigned)cdiv(wK.npw, 256), natom * c->pmax), dim3(256), 0,
-                               st, c->nlK.as<double>(), c->Y_K.as<double>(), wK.Fk, wK.npw, pj,
-                               c->d_plist, c->d_atype, c->d_apos, c->d_Fsign, -1,
-                               c->beta_K.as<z64>());
-        if (!mirror)
-            hipLaunchKernelGGL(k_nl_beta<double>,
-                               dim3((unsigned)cdiv(wKp.npw, 256), natom * c->pmax), dim3(256), 0,
-                               st, c->nlKp.as<double>(), c->Y_Kp.as<double>(), wKp.Fk, wKp.npw,
-                               pj, c->d_plist, c->d_atype, c->d_apos, c->d_Fsign, +1,
-                               c->beta_Kp.as<z64>());
-    }
-    HIP_TRY(hipGetLastError());
-    for (int side = 0; side < 2 && prec != LELPH_FP64; ++side)
-    {
-        if (skip_side(side)) continue;
-        const DevWfc& w = side == 0 ? wK : wKp;
-        const z64* A = side == 0 ? c->beta_K.as<z64>() : c->beta_Kp.as<z64>();
-        const z64* B = side == 0 ? c->wr_K.as<z64>() : c->wr_Kp.as<z64>();
-        z64* out = side == 0 ? c->bb_K.as<z64>() : c->bb_Kp.as<z64>();
-        const int conjB = side == 0 ? sK.conj_w : sKp.conj_w;
-        // bf16 contexts: FP32 operands on FP32 MFMA by default (c2: 0.16 ms
-        // per GEMM against 0.36 + 0.10 ms for the bf16 pieces, and closer:
-        // 1.3-1.9e-7 against 2.1-2.6e-7 of the non-local part alone); the
-        // non-local kernels run in the gaps between contractions, so their
-        // time counts.  nl_form 1: bf16 pieces, 3 of them and 6 products for
-        // both split precisions (the 2-piece form left 8.5e-6)
-        if (!nl32)
-            LELPH_TRY((nl_gemm_split<3, 6>(c, A, B, rows, ncol, w.npw, conjB, out, st)));
-        else
-        {
-            // FP32: beta from the FP64 tables, stored in FP32; psi rotated
-            // into FP32 by k_nl_geom
-            DBuf& b32 = side == 0 ? c->beta32_K : c->beta32_Kp;
-            DBuf& w32 = side == 0 ? c->wr32_K : c->wr32_Kp;
-            LELPH_TRY(b32.ensure(sizeof(c32) * (size_t)rows * npm));
-            hipLaunchKernelGGL(k_nl_beta<float>,
-                               dim3((unsigned)cdiv(w.npw, 256), natom * c->pmax), dim3(256), 0, st,
-                               side == 0 ? c->nlK.as<double>() : c->nlKp.as<double>(),
-                               side == 0 ? c->Y_K.as<double>() : c->Y_Kp.as<double>(), w.Fk,
-                               w.npw, pj, c->d_plist, c->d_atype, c->d_apos, c->d_Fsign,
-                               side == 0 ? -1 : +1, b32.as<c32>());
-            HIP_TRY(hipGetLastError());
-            const int64_t nchunks = cdiv(w.npw, CT_KC);
-            const int64_t tiles = cdiv(rows, GZ_MB) * cdiv(ncol, GZ_NB);
-            int64_t cps;
-            int nsplit;
-            pick_splits(tiles, nchunks, (int64_t)rows * ncol, &cps, &nsplit);
-            const size_t need = sizeof(z64) * (size_t)nsplit * rows * ncol;
-            if (need > c->bbpart.n && st != c->stream) HIP_TRY(hipStreamSynchronize(st));
-            LELPH_TRY(c->bbpart.ensure(need));
-            hipLaunchKernelGGL(k_zgemm_nt<float>, dim3((unsigned)tiles, (unsigned)nsplit),
-                               dim3(256), 0, st, b32.as<c32>(), w32.as<c32>(), rows, (int)ncol,
-                               w.npw, conjB, cps, c->bbpart.as<z64>());
-            hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv((int64_t)rows * ncol, 256)),
-                               dim3(256), 0, st, c->bbpart.as<z64>(), nsplit,
-                               (int64_t)rows * ncol, 1.0, out);
-            HIP_TRY(hipGetLastError());
-        }
-    }
-    for (int side = 0; side < 2 && prec == LELPH_FP64; ++side)
-    {
-        if (skip_side(side)) continue;
-        const DevWfc& w = side == 0 ? wK : wKp;
-        const z64* A = side == 0 ? c->beta_K.as<z64>() : c->beta_Kp.as<z64>();
-        const z64* B = side == 0 ? c->wr_K.as<z64>() : c->wr_Kp.as<z64>();
-        z64* out = side == 0 ? c->bb_K.as<z64>() : c->bb_Kp.as<z64>();
-        const int conjB = side == 0 ? sK.conj_w : sKp.conj_w;
-        const int64_t nchunks = cdiv(w.npw, CT_KC);
-        const int64_t tiles = cdiv(rows, GZ_MB) * cdiv(ncol, GZ_NB);
-        int64_t cps;
-        int nsplit;
-        pick_splits(tiles, nchunks, (int64_t)rows * ncol, &cps, &nsplit);
-        // the split count follows the side's npw: a larger partial buffer is
-        // allocated only once the previous pair's non-local part is done
-        const size_t need = sizeof(z64) * (size_t)nsplit * rows * ncol;
-        if (need > c->bbpart.n && st != c->stream) HIP_TRY(hipStreamSynchronize(st));
-        LELPH_TRY(c->bbpart.ensure(need));
-        hipLaunchKernelGGL(k_zgemm_nt<double>, dim3((unsigned)tiles, (unsigned)nsplit), dim3(256),
-                           0, st, A, B, rows, (int)ncol, w.npw, conjB, cps,
-                           c->bbpart.as<z64>());
-        hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv((int64_t)rows * ncol, 256)),
-                           dim3(256), 0, st, c->bbpart.as<z64>(), nsplit,
-                           (int64_t)rows * ncol, 1.0, out);
-        HIP_TRY(hipGetLastError());
-    }
-    if (mirror)
-        hipLaunchKernelGGL(k_nl_mirror, dim3((unsigned)cdiv((int64_t)rows * ncol, 256)),
-                           dim3(256), 0, st, c->bb_Kprev.as<z64>(), (int64_t)rows, ncol,
-                           c->bb_Kp.as<z64>());
-    if (close_k)
-        hipLaunchKernelGGL(k_nl_mirror, dim3((unsigned)cdiv((int64_t)rows * ncol, 256)),
-                           dim3(256), 0, st, c->bb_Khead.as<z64>(), (int64_t)rows, ncol,
-                           c->bb_K.as<z64>());
-    HIP_TRY(hipGetLastError());
-    const int64_t ne = (int64_t)natom * 3 * es;
-    z64* eb = ebuf_out ? ebuf_out : c->ebuf.as<z64>();
-    hipLaunchKernelGGL(k_nl_kkp, dim3((unsigned)cdiv(ne, 256)), dim3(256), 0, st,
-                       c->bb_K.as<z64>(), c->bb_Kp.as<z64>(), pj, c->d_plist, c->d_atype,
-                       c->d_socfac, c->d_fco, c->has_fco ? c->d_fco_off : nullptr, L.nspin,
-                       L.nbnds, L.nspinor, eb);
-    HIP_TRY(hipGetLastError());
-    if (c->nl_chain)
-    {
-        // this pair's K-side projections stay for the next pair of the chain
-        // (the kernels above are ordered before any later write on st)
-        LELPH_TRY(c->bb_Kprev.ensure(c->bb_K.n));
-        std::swap(c->bb_K.p, c->bb_Kprev.p);
-        std::swap(c->bb_K.n, c->bb_Kprev.n);
-        c->nl_prev_valid = true;
-        c->nl_prev_ik = pr.ikq;
-        c->nl_prev_sym = pr.kqsym;
-        // a chain's head keeps its K' projections for the cycle's close
-        if (!mirror)
-        {
-            LELPH_TRY(c->bb_Khead.ensure(c->bb_Kp.n));
-            std::swap(c->bb_Kp.p, c->bb_Khead.p);
-            std::swap(c->bb_Kp.n, c->bb_Khead.n);
-            c->nl_head_valid = true;
-            c->nl_head_ik = pr.ik;
-            c->nl_head_sym = pr.ksym;
-        }
-    }
-    if (ebuf_out) return LELPH_OK;
-    if (mode_after) HIP_TRY(hipStreamWaitEvent(st, mode_after, 0));
-    return nl_mode(c, eb, g, st);
+    return reduce_parts(c->part.as<z64>(), nsplit, gsz, 1.0 / (double)c->nf, g, c->stream);
 }
 
 // local part with split-product bf16 MFMA (split.hpp)
@@ -1209,10 +940,7 @@ static int run_local_split_t(lelph_ctx* c, const double* qpt, const lelph_pair& 
     HIP_TRY(hipGetLastError());
     const int nsplit = (int)ns;
     HIP_TRY(hipEventRecord(ev[2], c->stream));
-    hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(gsz, 256)), dim3(256), 0, c->stream,
-                       c->part.as<z64>(), nsplit, gsz, 1.0 / (double)c->nf, g);
-    HIP_TRY(hipGetLastError());
-    return LELPH_OK;
+    return reduce_parts(c->part.as<z64>(), nsplit, gsz, 1.0 / (double)c->nf, g, c->stream);
 }
 
 // The precision a context's contractions actually run in.  bf16x3 (two
@@ -1331,11 +1059,11 @@ static void free_ctx(lelph_ctx* c)
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     c->cv.release();
+    c->nl.release();
     c->cv_dv32.release();
     DBuf* bufs[] = {&c->dv64, &c->dv32, &c->eig_d, &c->vloc_tmp, &c->rot_tmp, &c->idx_k,
                     &c->idx_kq, &c->ph_k, &c->ph_kq, &c->box_k, &c->box_kq, &c->box_x, &c->part, &c->g,
-                    &c->gbatch, &c->presplit, &c->nlK, &c->nlKp, &c->Y_K, &c->Y_Kp, &c->wr_K, &c->wr_Kp,
-                    &c->beta_K, &c->beta_Kp, &c->bb_K, &c->bb_Kp, &c->bb_Kprev, &c->bb_Khead, &c->bbpart, &c->ebuf,
+                    &c->gbatch, &c->presplit,
                     &c->pl_cnt[0], &c->pl_cnt[1], &c->pl_off[0], &c->pl_off[1], &c->pl_cur[0],
                     &c->pl_cur[1], &c->pl_perm[0], &c->pl_perm[1], &c->dm_map, &c->dm_ph,
                     &c->dm_pos, &c->dm_wRS, &c->dm_wS2, &c->dm_part, &c->dm_out, &c->qr_dl,
@@ -1862,11 +1590,36 @@ static int ensure_events(lelph_ctx* c, int64_t npairs)
     return LELPH_OK;
 }
 
+// the windows of a batch's pairs in the order they are worked on, groups of
+// `step` pairs
+static void nl_plan(lelph_ctx* c, const lelph_pair* pairs, const std::vector<int64_t>& order,
+                    int64_t step)
+{
+    c->nl_step = nl_window(c, step, (int64_t)order.size());
+    c->nl_win.clear();
+    for (size_t i = 0; i < order.size(); ++i)
+    {
+        if (i % (size_t)c->nl_step == 0) c->nl_win.emplace_back();
+        c->nl_win.back().add(pairs[order[i]]);
+    }
+}
+
+// non-local part of pairs p0 .. p0 + n - 1 of that order into their g on the
+// second stream; a window's sides are projected with its first group
+static int nl_batch(lelph_ctx* c, int64_t p0, int64_t n, z64* g, hipEvent_t after)
+{
+    const int64_t w = p0 / c->nl_step;
+    if (p0 % c->nl_step == 0)
+        LELPH_TRY(nl_sides(c, c->nl, c->nl.desc, c->nl_win[(size_t)w], true, c->nl_stream));
+    return nl_add(c, c->nl, p0 - w * c->nl_step, n, g, c->nl_stream, after);
+}
+
 // local (+ non-local) of one pair into device g; events ev[0..4], ev[4]
-// marking the end of both parts.  overlap: the non-local part runs on
-// nl_stream, beside this pair's local part and the next pair's boxes.
+// marking the end of both parts.  batch_pos: position in the batch (nl_plan);
+// its non-local part runs on nl_stream, beside this pair's local part and the
+// next pair's boxes.
 static int gkq_device(lelph_ctx* c, const double* qpt, const lelph_pair& pr, int local,
-                      int nonloc, z64* g, hipEvent_t* ev, bool overlap = false)
+                      int nonloc, z64* g, hipEvent_t* ev, int64_t batch_pos = -1)
 {
     HIP_TRY(hipEventRecord(ev[0], c->stream));
     if (local)
@@ -1877,13 +1630,19 @@ static int gkq_device(lelph_ctx* c, const double* qpt, const lelph_pair& pr, int
         HIP_TRY(hipEventRecord(ev[2], c->stream));
     }
     HIP_TRY(hipEventRecord(ev[3], c->stream));
-    if (nonloc && overlap)
+    if (nonloc && batch_pos >= 0)
     {
-        LELPH_TRY(run_nonlocal(c, pr, g, c->nl_stream, ev[3]));
+        LELPH_TRY(nl_batch(c, batch_pos, 1, g, ev[3]));
         HIP_TRY(hipEventRecord(ev[4], c->nl_stream));
         return LELPH_OK;
     }
-    if (nonloc) LELPH_TRY(run_nonlocal(c, pr, g, c->stream, nullptr));
+    if (nonloc)
+    {
+        NlWindow w;
+        w.add(pr);
+        LELPH_TRY(nl_sides(c, c->nl, c->nl.desc, w, true, c->stream));
+        LELPH_TRY(nl_add(c, c->nl, 0, 1, g, c->stream, nullptr));
+    }
     HIP_TRY(hipEventRecord(ev[4], c->stream));
     return LELPH_OK;
 }
@@ -2036,9 +1795,7 @@ static int conv_batch(lelph_ctx* c, const ConvGeo& geo, const double* qpt, int64
         return LELPH_OK;
     };
     c->box_sides = chain_sides(pairs, order);
-    c->nl_chain = true;
-    c->nl_prev_valid = false;
-    c->nl_head_valid = false;
+    if (non_loc) nl_plan(c, pairs, order, np);
     std::vector<lelph_pair> grp((size_t)np);
     int64_t landed = 0;
     auto body = [&](int64_t gi) -> int {
@@ -2052,8 +1809,7 @@ static int conv_batch(lelph_ctx* c, const ConvGeo& geo, const double* qpt, int64
         HIP_TRY(hipEventRecord(ev[3], c->stream));
         if (non_loc)
         {
-            for (int64_t i = 0; i < n; ++i)
-                LELPH_TRY(run_nonlocal(c, grp[i], g + i * gsz, c->nl_stream, ev[3]));
+            LELPH_TRY(nl_batch(c, p0, n, g, ev[3]));
             HIP_TRY(hipEventRecord(ev[4], c->nl_stream));
         }
         else
@@ -2068,9 +1824,6 @@ static int conv_batch(lelph_ctx* c, const ConvGeo& geo, const double* qpt, int64
     };
     int st = LELPH_OK;
     for (int64_t gi = 0; gi < ngroups && st == LELPH_OK; ++gi) st = body(gi);
-    c->nl_chain = false;
-    c->nl_prev_valid = false;
-    c->nl_head_valid = false;
     if (st != LELPH_OK)
     {
         (void)hipStreamSynchronize(c->nl_stream);
@@ -2127,16 +1880,14 @@ int lelph_gkq_batch(lelph_ctx* c, const double qpt[3], int64_t npairs, const lel
     c->box_prev_valid = false;
     c->box_head = nullptr;
     c->box_sides = 0;
-    c->nl_chain = true;
-    c->nl_prev_valid = false;
-    c->nl_head_valid = false;
+    if (non_loc) nl_plan(c, pairs, order, 1);
     int st = LELPH_OK;
     int64_t landed = 0;
     for (int64_t n = 0; n < npairs && st == LELPH_OK; ++n)
     {
         const int64_t i = order[n];
         st = gkq_device(c, qpt, pairs[i], 1, non_loc, c->gbatch.as<z64>() + i * gsz,
-                        c->evs.data() + 5 * i, true);
+                        c->evs.data() + 5 * i, n);
         if (st != LELPH_OK) break;
         if (n >= LELPH_OUT_SLOTS)
         {
@@ -2153,9 +1904,6 @@ int lelph_gkq_batch(lelph_ctx* c, const double qpt[3], int64_t npairs, const lel
     c->box_reuse = false;
     c->box_prev_valid = false;
     c->box_head = nullptr;
-    c->nl_chain = false;
-    c->nl_prev_valid = false;
-    c->nl_head_valid = false;
     if (st != LELPH_OK)
     {
         (void)hipStreamSynchronize(c->nl_stream);
@@ -2192,7 +1940,7 @@ struct MultiPair
     int64_t close = -1; // the chain head whose psi_k box is its psi_k+q box
     int g0[3] = {0, 0, 0}; // umklapp vector of its k+q side
     void* kbox = nullptr;  // its psi_k box: box_k, or the linked pair's box_kq
-    DBuf box_k, box_kq, part, ebuf;
+    DBuf box_k, box_kq, part;
 };
 } // namespace
 
@@ -2219,6 +1967,16 @@ struct lelph_multi
         std::vector<lelph_pair> pairs;
     };
     std::vector<ConvCell> conv;
+    // non-local parts: per cell its buffers (the sums of all its pairs) and
+    // per window of pairs the sides and their descriptors
+    struct NlCell
+    {
+        NlBufs bufs;
+        std::vector<NlWindow> win;
+        std::vector<DBuf> desc;
+        int64_t step = 1;
+    };
+    std::vector<NlCell> nlc;
     std::vector<DBuf> gdev;    // per cell: (npairs, nmodes, nspin, nb, nb) complex128
     std::vector<void*> ghost;  // per cell: pinned copy of gdev
     std::vector<size_t> gbytes;
@@ -2234,8 +1992,8 @@ struct lelph_multi
     std::vector<Queue> queues;
     DBuf counter;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-    // the non-local parts run on a second stream: forked at the start,
-    // their mode rotations wait for the reductions, joined before the copy
+    // they run on a second stream: forked at the start, their mode rotations
+    // wait for the reductions, joined before the copy
     hipStream_t nl = nullptr;
     hipEvent_t fork = nullptr, reduced = nullptr, joined = nullptr;
     double ms[4] = {0, 0, 0, 0};
@@ -2313,29 +2071,17 @@ static int multi_enqueue(lelph_multi* m, bool timed)
         {
             HIP_TRY(hipEventRecord(m->fork, m->stream));
             HIP_TRY(hipStreamWaitEvent(m->nl, m->fork, 0));
-            // along each cell's chains, as lelph_gkq_batch: a pair's K'
-            // projections are the previous pair's K ones, mirrored
-            for (lelph_ctx* c : m->ctx)
+            for (size_t i = 0; i < m->ctx.size(); ++i)
             {
-                c->nl_chain = true;
-                c->nl_prev_valid = false;
-                c->nl_head_valid = false;
+                auto& nc = m->nlc[i];
+                const int64_t one = nl_sum_size(m->ctx[i]);
+                for (size_t k = 0; k < nc.win.size(); ++k)
+                {
+                    LELPH_TRY(nl_sides(m->ctx[i], nc.bufs, nc.desc[k], nc.win[k], first, m->nl));
+                    LELPH_TRY(nl_sums(m->ctx[i], nc.bufs, 0, (int64_t)nc.win[k].kk.size() / 2,
+                                      nc.bufs.ebuf.as<z64>() + (int64_t)k * nc.step * one, m->nl));
+                }
             }
-            int nst = LELPH_OK;
-            for (int64_t bi : m->border)
-            {
-                MultiPair& p = m->pairs[(size_t)bi];
-                nst = run_nonlocal(m->ctx[p.cell], p.pr, nullptr, m->nl, nullptr,
-                                   p.ebuf.as<z64>());
-                if (nst != LELPH_OK) break;
-            }
-            for (lelph_ctx* c : m->ctx)
-            {
-                c->nl_chain = false;
-                c->nl_prev_valid = false;
-                c->nl_head_valid = false;
-            }
-            LELPH_TRY(nst);
         }
         // every pair's psi_k+q box into its own slot, along each cell's
         // k -> k+q chains: a linked pair's psi_k box is the k+q box of the
@@ -2396,18 +2142,17 @@ static int multi_enqueue(lelph_multi* m, bool timed)
             if (m->conv[p.cell].on) continue;
             lelph_ctx* c = m->ctx[p.cell];
             z64* g = m->gdev[p.cell].as<z64>() + p.index * p.gsz;
-            hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(p.gsz, 256)), dim3(256), 0,
-                               m->stream, p.part.as<z64>(), p.nsplit, p.gsz, 1.0 / (double)c->nf,
-                               g);
-            HIP_TRY(hipGetLastError());
+            LELPH_TRY(reduce_parts(p.part.as<z64>(), p.nsplit, p.gsz, 1.0 / (double)c->nf, g,
+                                   m->stream));
         }
         if (m->non_loc)
         {
             HIP_TRY(hipEventRecord(m->reduced, m->stream));
             HIP_TRY(hipStreamWaitEvent(m->nl, m->reduced, 0));
-            for (auto& p : m->pairs)
-                LELPH_TRY(nl_mode(m->ctx[p.cell], p.ebuf.as<z64>(),
-                                  m->gdev[p.cell].as<z64>() + p.index * p.gsz, m->nl));
+            for (size_t i = 0; i < m->ctx.size(); ++i)
+                if (m->npairs[i])
+                    LELPH_TRY(nl_modes(m->ctx[i], m->nlc[i].bufs.ebuf.as<z64>(), m->npairs[i],
+                                       m->gdev[i].as<z64>(), m->nl));
             HIP_TRY(hipEventRecord(m->joined, m->nl));
             HIP_TRY(hipStreamWaitEvent(m->stream, m->joined, 0));
         }
@@ -2509,12 +2254,16 @@ static void multi_free(lelph_multi* m)
         p.box_k.release();
         p.box_kq.release();
         p.part.release();
-        p.ebuf.release();
     }
     for (auto& cc : m->conv)
     {
         cc.bufs.release();
         for (auto& d : cc.desc) d.release();
+    }
+    for (auto& nc : m->nlc)
+    {
+        nc.bufs.release();
+        for (auto& d : nc.desc) d.release();
     }
     for (auto& g : m->gdev) g.release();
     for (void* h : m->ghost)
@@ -2603,6 +2352,20 @@ static int multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
             int st = ensure_dv32(c);
             if (st != LELPH_OK) return fail(st);
         }
+        m->nlc.emplace_back();
+        if (m->non_loc && npairs[i])
+        {
+            auto& nc = m->nlc.back();
+            nc.step = nl_window(c, 1, npairs[i]);
+            for (int64_t j = 0; j < npairs[i]; ++j)
+            {
+                if (j % nc.step == 0) nc.win.emplace_back();
+                nc.win.back().add(pairs[i][j]);
+            }
+            nc.desc.resize(nc.win.size());
+            if (nc.bufs.ebuf.ensure(sizeof(z64) * (size_t)(nl_sum_size(c) * npairs[i])))
+                return fail(LELPH_ERR_ALLOC);
+        }
         if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(LELPH_ERR_HIP);
         const lelph_lattice& L = c->lat;
         const int64_t gsz = (int64_t)L.nmodes * L.nspin * L.nbnds * L.nbnds;
@@ -2624,7 +2387,6 @@ static int multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
             p.tiles = ct_tiles(shape, L.nmodes, L.nbnds);
             pick_splits(tiles * L.nspin, nchunks, gsz, &p.cps, &p.nsplit, c->tune.split_target);
             p.bb = bb;
-            const int64_t es = (int64_t)L.nspin * L.nbnds * L.nbnds;
             // the k+q side's umklapp vector (it shifts the box a linked
             // pair takes over)
             SideGeom gkq, gk;
@@ -2636,9 +2398,8 @@ static int multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
                 return fail(gs);
             }
             for (int d = 0; d < 3; ++d) p.g0[d] = (int)std::lrint(gkq.G0c[d]);
-            if ((!cc.on && (p.box_kq.ensure(bb) ||
-                            p.part.ensure(sizeof(z64) * (size_t)(p.nsplit * gsz)))) ||
-                (non_loc && p.ebuf.ensure(sizeof(z64) * (size_t)(3 * L.natom * es))))
+            if (!cc.on && (p.box_kq.ensure(bb) ||
+                           p.part.ensure(sizeof(z64) * (size_t)(p.nsplit * gsz))))
             {
                 m->pairs.push_back(p);
                 return fail(LELPH_ERR_ALLOC);
@@ -2907,10 +2668,8 @@ int lelph_electronic_reps(lelph_ctx* c, const double Rsym[9], const double tauR[
                            0, c->stream, c->dm_wS2.as<z64>() + is * nb * Lk,
                            c->dm_wRS.as<z64>() + is * nb * Lk, nb, nb, Lk, 0, cps,
                            c->dm_part.as<z64>());
-        hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv((int64_t)nb * nb, 256)), dim3(256),
-                           0, c->stream, c->dm_part.as<z64>(), nsplit, (int64_t)nb * nb, 1.0,
-                           c->dm_out.as<z64>() + (int64_t)is * nb * nb);
-        HIP_TRY(hipGetLastError());
+        LELPH_TRY(reduce_parts(c->dm_part.as<z64>(), nsplit, (int64_t)nb * nb, 1.0,
+                               c->dm_out.as<z64>() + (int64_t)is * nb * nb, c->stream));
     }
     HIP_TRY(hipMemcpyAsync(Dkmn, c->dm_out.p, sizeof(z64) * L.nspin * nb * nb,
                            hipMemcpyDeviceToHost, c->stream));
