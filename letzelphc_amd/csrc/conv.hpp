@@ -462,11 +462,11 @@ struct LnTable
         return ln_tw<SIGN>(W, j * k);
     }
 };
-template <int R2>
+template <int R2, typename T>
 struct LnLds // copied to LDS, [k][j]
 {
-    const z64* tw;
-    __device__ __forceinline__ z64 operator()(int j, int k) const { return tw[k * R2 + j]; }
+    const cpx<T>* tw;
+    __device__ __forceinline__ cpx<T> operator()(int j, int k) const { return tw[k * R2 + j]; }
 };
 struct LnHeld
 {
@@ -599,8 +599,7 @@ __device__ __forceinline__ void ln_exchange(const cpx<A>* x, cpx<A>* v, char* Sw
 // LR rows at a time through both steps, the next rows' psi loaded before the
 // second step of the current ones.
 template <typename T, bool TWO, int R1, int R2>
-__device__ inline void plane_z_rows(const ConvSrc<T>& q, int Ny, const z64* __restrict__ W,
-                                    char* S, cpx<T>* P, int prow, const unsigned short* yad,
+__device__ inline void plane_z_rows(const ConvSrc<T>& q, int Ny, const LnLds<R2, T>& tw, char* S, cpx<T>* P, int prow, const unsigned short* yad,
                                     const short* zc, int NW, int tid)
 {
     constexpr int LR = ln_rows(R2), N = R1 * R2, M = TWO ? 2 : 1;
@@ -612,26 +611,30 @@ __device__ inline void plane_z_rows(const ConvSrc<T>& q, int Ny, const z64* __re
     auto row_of = [&](int y) { return min(y + r, Ny - 1) * N; };
     auto fetch = [&](int y) {
         ln_load<R1, R2>(p[0], q.p0 + row_of(y), j);
-        if constexpr (TWO) ln_load<R1, R2>(p[1], q.p1 + row_of(y), j);
+        if constexpr (TWO)
+            ln_load<R1, R2>(p[1], q.p1 + row_of(y), j);
     };
     fetch(wave * LR);
     for (int y0 = wave * LR; y0 < Ny; y0 += NW * LR)
     {
         cpx<T> x[R1], v[R2];
+        if constexpr (TWO)
         {
-            cpx<T> d[M][R1];
-            ln_load<R1, R2>(d[0], q.v0 + row_of(y0), j);
-            if constexpr (TWO) ln_load<R1, R2>(d[1], q.v1 + row_of(y0), j);
+            cpx<T> e[2][R1]; // no registers to load these ahead
+            ln_load<R1, R2>(e[0], q.v0 + row_of(y0), j);
+            ln_load<R1, R2>(e[1], q.v1 + row_of(y0), j);
 #pragma unroll
-            for (int i = 0; i < R1; ++i)
-            {
-                x[i] = cmul(d[0][i], p[0][i]);
-                if constexpr (TWO) x[i] = cadd(x[i], cmul(d[1][i], p[1][i]));
-            }
+            for (int i = 0; i < R1; ++i) x[i] = cadd(cmul(e[0][i], p[0][i]), cmul(e[1][i], p[1][i]));
+        }
+        else
+        {
+            ln_load<R1, R2>(x, q.v0 + row_of(y0), j);
+#pragma unroll
+            for (int i = 0; i < R1; ++i) x[i] = cmul(x[i], p[0][i]);
         }
         Rdft<T, -1, R1>::run(x);
 #pragma unroll
-        for (int k = 1; k < R1; ++k) x[k] = cmul(x[k], to<T>(ln_tw<-1>(W, j * k)));
+        for (int k = 1; k < R1; ++k) x[k] = cmul(x[k], tw(j, k));
         if (y0 + NW * LR < Ny) fetch(y0 + NW * LR);
         ln_exchange<T, R1, R2>(x, v, Sw, r, j, rd, k1);
         Rdft<T, -1, R2>::run(v);
@@ -735,11 +738,13 @@ struct ConvArgs
     int rows_per_block;
 };
 
-// LDS of a plane block: exchange rows, plane buffer, y addresses, kept columns
+// LDS of a plane block: exchange rows, plane buffer, y addresses, kept
+// columns, twiddles of both axes
 struct PlaneLds
 {
     int rows;  // bytes of the exchange rows
     int prow;  // elements of a plane column
+    int tw;    // offset of the twiddles
     size_t bytes;
 };
 
@@ -749,8 +754,10 @@ static inline PlaneLds plane_lds(int R1y, int R2y, int R1z, int R2z, int nzk, in
     PlaneLds l;
     l.rows = ((NT / 64) * ln_space(R2z) * ln_row_bytes<T>(R1z, R2z) + 15) & ~15;
     l.prow = ln_prow(R1y, R2y);
-    l.bytes = (size_t)l.rows + sizeof(cpx<T>) * (size_t)nzk * l.prow +
-              2 * (size_t)(R1y * R2y + R1z * R2z + nzk * R1y * R2y) + 16;
+    l.tw = (int)(((size_t)l.rows + sizeof(cpx<T>) * (size_t)nzk * l.prow +
+                  2 * (size_t)(R1y * R2y + R1z * R2z + nzk * R1y * R2y) + 15) &
+                 ~(size_t)15);
+    l.bytes = (size_t)l.tw + sizeof(cpx<T>) * (size_t)(R1y * R2y + R1z * R2z);
     return l;
 }
 
@@ -831,8 +838,8 @@ constexpr int rx_class(int R1, int R2) { return R1 <= 10 && R2 <= 12 ? 0 : 1; }
 
 struct PlaneArgs
 {
-    int s_bytes, prow; // of PlaneLds
-    int R1y, R2y;
+    int s_bytes, prow, tw; // of PlaneLds
+    int R1y, R2y, R2z;
 };
 
 // block -> (x, inner, outer): all blocks of an x plane on one XCD (block b
@@ -928,7 +935,10 @@ constexpr int plane_threads(int cls)
     return cls == 0 ? (sizeof(T) == 8 ? (TWO ? 256 : 512) : 768) : 256;
 }
 
-// any compiled (Ny, Nz)
+// any compiled (Ny, Nz).  Twiddles in LDS: read from the table per line they
+// were a third of the address cycles (36^3 spinor, FP32: 1.58 -> 1.41 ms per
+// 8 pairs; 45 x 108 planes, FP64: 1 %).  Loading dV a group ahead beside psi
+// gains nothing here and costs 5 % in k_conv_square in FP64.
 template <typename T, bool TWO, int CLS>
 __global__ __launch_bounds__((plane_threads<T, TWO>(CLS))) void k_conv_plane(
     const ConvPair* __restrict__ pairs, const SphSide* __restrict__ sides, ConvArgs a,
@@ -943,6 +953,12 @@ __global__ __launch_bounds__((plane_threads<T, TWO>(CLS))) void k_conv_plane(
     unsigned short* yad = reinterpret_cast<unsigned short*>(P + a.nzk_max * pa.prow);
     short* zl = reinterpret_cast<short*>(yad + Ny);
     unsigned short* sl = reinterpret_cast<unsigned short*>(zl + Nz);
+    cpx<T>* twy = reinterpret_cast<cpx<T>*>(cv_smem + pa.tw);
+    cpx<T>* twz = twy + Ny;
+    for (int f = threadIdx.x; f < Ny; f += blockDim.x)
+        twy[f] = to<T>(ln_tw<-1>(Wy, (f / pa.R2y) * (f % pa.R2y)));
+    for (int f = threadIdx.x; f < Nz; f += blockDim.x)
+        twz[f] = to<T>(ln_tw<-1>(Wz, (f / pa.R2z) * (f % pa.R2z)));
     plane_tables(jb.zc, Ny, Nz, false, pa.R1y, pa.R2y, yad, zl);
     plane_sticks(jb.smap, jb.nzk * Ny, sl);
     __syncthreads();
@@ -958,7 +974,8 @@ __global__ __launch_bounds__((plane_threads<T, TWO>(CLS))) void k_conv_plane(
 #define CV_CASE(L, A, B)                                                                          \
     case L:                                                                                       \
         if constexpr (rx_class(A, B) <= CLS)                                                      \
-            plane_z_rows<T, TWO, A, B>(q, Ny, Wz, cv_smem, P, pa.prow, yad, zl, NW, tid);         \
+            plane_z_rows<T, TWO, A, B>(q, Ny, LnLds<B, T>{twz}, cv_smem, P, pa.prow, yad, zl, NW, \
+                                       tid);                                                      \
         break;
             RX_LENGTHS(CV_CASE)
 #undef CV_CASE
@@ -971,7 +988,7 @@ __global__ __launch_bounds__((plane_threads<T, TWO>(CLS))) void k_conv_plane(
 #define CV_CASE(L, A, B)                                                                          \
     case L:                                                                                       \
         if constexpr (rx_class(A, B) <= CLS)                                                      \
-            plane_y_out<T, A, B>(P, jb.nzk, LnTable<-1>{Wy}, sl, out, NW, tid);                    \
+            plane_y_out<T, A, B>(P, jb.nzk, LnLds<B, T>{twy}, sl, out, NW, tid);                  \
         break;
             RX_LENGTHS(CV_CASE)
 #undef CV_CASE
@@ -1016,13 +1033,13 @@ __global__ __launch_bounds__(64 * NW, (sizeof(T) == 4 ? 3 : 1)) void k_conv_squa
     constexpr bool TL = sq_tw_lds(R1), TZ = sizeof(T) == 4;
     z64 tw[TL ? 1 : R1];
     cpx<T> tz[TZ ? R1 : 1];
-    z64* twl = reinterpret_cast<z64*>(
+    cpx<T>* twl = reinterpret_cast<cpx<T>*>(
         cv_smem + SB + ((sizeof(cpx<T>) * (size_t)a.nzk_max * PR + 15) & ~(size_t)15) +
         ((2 * (size_t)a.nzk_max * N + 15) & ~(size_t)15));
     if constexpr (TL)
     {
         for (int f = threadIdx.x; f < N; f += 64 * NW)
-            twl[f] = ln_tw<-1>(W, (f / R2) * (f % R2));
+            twl[f] = to<T>(ln_tw<-1>(W, (f / R2) * (f % R2)));
         lds_barrier();
     }
     else
@@ -1033,7 +1050,7 @@ __global__ __launch_bounds__(64 * NW, (sizeof(T) == 4 ? 3 : 1)) void k_conv_squa
         for (int k = 1; k < R1; ++k) tz[k] = to<T>(ln_tw<-1>(W, j * k));
     auto twid = [&]() {
         if constexpr (TL)
-            return LnLds<R2>{twl};
+            return LnLds<R2, T>{twl};
         else
             return LnHeld{tw};
     };
@@ -1058,20 +1075,16 @@ __global__ __launch_bounds__(64 * NW, (sizeof(T) == 4 ? 3 : 1)) void k_conv_squa
             if (y0 < N) // uniform over the wave
             {
                 cpx<T> x[R1], v[R2];
-                {
-                    cpx<T> e[R1];
-                    if (g >= KG) load(e, dv + row_of(g));
+                if (g >= KG) load(x, dv + row_of(g));
 #pragma unroll
-                    for (int i = 0; i < R1; ++i)
-                        x[i] = cmul(g < KG ? d[g < KG ? g : 0][i] : e[i], p[i]);
-                }
+                for (int i = 0; i < R1; ++i) x[i] = cmul(g < KG ? d[g < KG ? g : 0][i] : x[i], p[i]);
                 Rdft<T, -1, R1>::run(x);
 #pragma unroll
                 for (int k = 1; k < R1; ++k) 
                     if constexpr (TZ)
                         x[k] = cmul(x[k], tz[k]);
                     else
-                        x[k] = cmul(x[k], twid()(j, k));
+                        x[k] = cmul(x[k], to<T>(twid()(j, k)));
                 // the next rows that this wave has, or the next set's first
                 const bool more = g + 1 < G && y0 + NW * LR < N;
                 load(p, (more ? q.p0 : qn.p0) + row_of(more ? g + 1 : 0));

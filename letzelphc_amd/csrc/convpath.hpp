@@ -26,8 +26,9 @@ struct ConvGeo
 // bytes of line buffers (the planes' output) that a launch may fill.  More
 // than the 256 MB last-level cache on purpose: fewer, longer launches and
 // more sets per psi plane outweigh what the x step finds cached (96^3, FP64,
-// per pair: 39.7 ms with 128 MB, 35.6 with 512, 34.6 with 1000)
-static const int64_t CONV_LINE_BYTES = 512ll << 20;
+// per pair: 39.7 ms with 128 MB, 35.6 with 512, 34.6 with 1000; a slab's 36
+// pairs 15.1 ms with 512, 14.1 with 1024)
+static const int64_t CONV_LINE_BYTES = 1024ll << 20;
 // modes of a launch that share a psi plane in L2 (4: 3 % slower in FP32, 16:
 // no gain), sets that a block takes in turn (32: the blocks of one psi plane
 // drift apart and miss, 3 %; 4: 2 % in starting blocks)
@@ -117,7 +118,7 @@ static bool conv_geo(const lelph_ctx* c, ConvGeo* g)
         g->sqlds = (((size_t)nw * ln_space(r2) * rb + 15) & ~(size_t)15) +
                    ((item * (size_t)g->nzk * ln_prow(r1, r2) + 15) & ~(size_t)15) +
                    ((2 * (size_t)g->nzk * r1 * r2 + 15) & ~(size_t)15) +
-                   (sq_tw_lds(r1) ? sizeof(z64) * r1 * r2 : 0);
+                   (sq_tw_lds(r1) ? item * r1 * r2 : 0);
         g->square = g->sqlds <= 160 * 1024;
     }
     if (!conv_plane_shape(*g, item, cls == 0 ? 512 : 256, false, &g->box)) return false;
@@ -309,12 +310,14 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
         dim3(tiles, (unsigned)cdiv(geo.nrows, ba.rows_per_block), (unsigned)nk), st, ds + np, ba,
         Wx));
     const int64_t nx8 = 8 * cdiv(Nx, 8);
-    PlaneArgs pb{geo.box.lds.rows, geo.box.lds.prow, geo.r1[1], geo.r2[1]};
+    PlaneArgs pb{geo.box.lds.rows, geo.box.lds.prow, geo.box.lds.tw,
+                 geo.r1[1], geo.r2[1], geo.r2[2]};
     LELPH_TRY(conv_box_plane_launch<T>(geo.box, nx8 * geo.nrows * nk, st, ds + np, ba, pb, Wy,
                                        Wz));
     if (ev) HIP_TRY(hipEventRecord(ev[1], st));
     // dV psi to the sphere, a chunk of modes at a time
-    PlaneArgs pc{geo.conv.lds.rows, geo.conv.lds.prow, geo.r1[1], geo.r2[1]};
+    PlaneArgs pc{geo.conv.lds.rows, geo.conv.lds.prow, geo.conv.lds.tw,
+                 geo.r1[1], geo.r2[1], geo.r2[2]};
     for (int64_t vs = 0; vs < cdiv(L.nmodes, nv) * cdiv(geo.nrows, nset); ++vs)
     {
         // sets outside, modes inside: the psi boxes of the sets stay cached
