@@ -76,20 +76,6 @@ __global__ void k_dm_side1(const double* __restrict__ gvec, int64_t npw, DmGeom 
     ph[3 * g + 2] = dm_phase(geo.Rkcrys, g2, geo.tau2c);
 }
 
-// k2 side, per G: partner position in the k1 list (-1 if none)
-__global__ void k_dm_side2(const double* __restrict__ gvec, int64_t npw, DmGeom geo, int Nx,
-                           int Ny, int Nz, const int* __restrict__ map, int* __restrict__ pos)
-{
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= npw) return;
-    const double G[3] = {gvec[3 * g], gvec[3 * g + 1], gvec[3 * g + 2]};
-    double g3[3];
-    dm_rot(geo.M3, G, g3);
-    for (int i = 0; i < 3; ++i) g3[i] += geo.ulmc[i];
-    const int b = dm_boxidx(g3, Nx, Ny, Nz);
-    pos[g] = b < 0 ? -1 : map[b];
-}
-
 __device__ inline void dm_su2(const z64* su, z64& u, z64& d)
 {
     const z64 u2 = cadd(cmul(u, su[0]), cmul(d, su[1]));
@@ -98,62 +84,90 @@ __device__ inline void dm_su2(const z64* su, z64& u, z64& d)
     d = d2;
 }
 
-// wRS[set][sp][g]: U(R) U(S1) applied to the k1 coefficients (elec_reps.c:310-328)
-__global__ void k_dm_rot1(const z64* __restrict__ w1, int64_t nsets, int nspinor, int64_t npw,
-                          const z64* __restrict__ ph, DmGeom geo, z64* __restrict__ wRS)
+// what a D matrix finds cleared: no partner anywhere, zero where a partner is
+// missing, no error.  One launch for what were three fills: a D matrix of a
+// small crystal is bound by its launches (45 x 45 x 108 slab, 40 bands, two D
+// matrices and a rotated g per point: 145 -> 119 us with 5 launches per
+// matrix, not 9).
+__global__ void k_dm_clear(int* __restrict__ map, int64_t nf, z64* __restrict__ wS2, int64_t n,
+                           int* __restrict__ err)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nsets * npw) return;
-    const int64_t s = t / npw, g = t - s * npw;
-    const z64* w = w1 + s * nspinor * npw;
-    z64 u = w[g], d = nspinor == 2 ? w[npw + g] : z64{0, 0};
-    if (nspinor == 2) dm_su2(geo.su1, u, d);
-    u = cmul(u, ph[3 * g]);
-    d = cmul(d, ph[3 * g]);
-    if (geo.tr1)
-    {
-        u.y = -u.y;
-        d.y = -d.y;
-    }
-    if (nspinor == 2) dm_su2(geo.suR, u, d);
-    u = cmul(u, ph[3 * g + 1]);
-    d = cmul(d, ph[3 * g + 1]);
-    if (geo.trR)
-    {
-        u.y = -u.y;
-        d.y = -d.y;
-    }
-    z64* o = wRS + s * nspinor * npw;
-    o[g] = u;
-    if (nspinor == 2) o[npw + g] = d;
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (int64_t t = t0; t < nf; t += step) map[t] = -1;
+    for (int64_t t = t0; t < n; t += step) wS2[t] = {0, 0};
+    if (t0 == 0) *err = 0;
 }
 
-// wS2[set][sp][pos]: the k2 coefficients moved to their k1 partners, U(S2),
-// translation, and the sandwich conjugate (elec_reps.c:329-373); the
-// destination is zeroed beforehand
-__global__ void k_dm_rot2(const z64* __restrict__ w2, int64_t nsets, int nspinor, int64_t npw2,
-                          int64_t npw1, const int* __restrict__ pos, const z64* __restrict__ ph,
-                          DmGeom geo, z64* __restrict__ wS2)
+// both rotations of DM_SETS sets per thread.  blockIdx.z 0: wRS[set][sp][g],
+// U(R) U(S1) applied to the k1 coefficients (elec_reps.c:310-328); 1:
+// wS2[set][sp][partner], the k2 coefficients moved to their k1 partners,
+// U(S2), translation, and the sandwich conjugate (elec_reps.c:329-373).
+#define DM_SETS 4
+__global__ __launch_bounds__(128) void k_dm_rot(
+    const z64* __restrict__ w1, int64_t npw1, const double* __restrict__ gvec2,
+    const z64* __restrict__ w2, int64_t npw2, int64_t nsets, int nspinor, DmGeom geo, int Nx,
+    int Ny, int Nz, const int* __restrict__ map, const z64* __restrict__ ph,
+    z64* __restrict__ wRS, z64* __restrict__ wS2)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nsets * npw2) return;
-    const int64_t s = t / npw2, g = t - s * npw2;
-    const int p = pos[g];
-    if (p < 0) return;
-    const z64* w = w2 + s * nspinor * npw2;
-    z64 u = w[g], d = nspinor == 2 ? w[npw2 + g] : z64{0, 0};
-    if (nspinor == 2) dm_su2(geo.su2, u, d);
-    const z64 f = ph[3 * p + 2];
-    u = cmul(u, f);
-    d = cmul(d, f);
-    if (!geo.tr2)
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t s0 = (int64_t)blockIdx.y * DM_SETS;
+    const int64_t s1 = s0 + DM_SETS < nsets ? s0 + DM_SETS : nsets;
+    if (blockIdx.z == 0)
     {
-        u.y = -u.y;
-        d.y = -d.y;
+        if (g >= npw1) return;
+        const z64 f1 = ph[3 * g], f2 = ph[3 * g + 1];
+        for (int64_t s = s0; s < s1; ++s)
+        {
+            const z64* w = w1 + s * nspinor * npw1;
+            z64 u = w[g], d = nspinor == 2 ? w[npw1 + g] : z64{0, 0};
+            if (nspinor == 2) dm_su2(geo.su1, u, d);
+            u = cmul(u, f1);
+            d = cmul(d, f1);
+            if (geo.tr1)
+            {
+                u.y = -u.y;
+                d.y = -d.y;
+            }
+            if (nspinor == 2) dm_su2(geo.suR, u, d);
+            u = cmul(u, f2);
+            d = cmul(d, f2);
+            if (geo.trR)
+            {
+                u.y = -u.y;
+                d.y = -d.y;
+            }
+            z64* o = wRS + s * nspinor * npw1;
+            o[g] = u;
+            if (nspinor == 2) o[npw1 + g] = d;
+        }
+        return;
     }
-    z64* o = wS2 + s * nspinor * npw1;
-    o[p] = u;
-    if (nspinor == 2) o[npw1 + p] = d;
+    if (g >= npw2) return;
+    const double G[3] = {gvec2[3 * g], gvec2[3 * g + 1], gvec2[3 * g + 2]};
+    double g3[3];
+    dm_rot(geo.M3, G, g3);
+    for (int i = 0; i < 3; ++i) g3[i] += geo.ulmc[i];
+    const int b = dm_boxidx(g3, Nx, Ny, Nz);
+    const int p = b < 0 ? -1 : map[b]; // position in the k1 list
+    if (p < 0) return;
+    const z64 f = ph[3 * (int64_t)p + 2];
+    for (int64_t s = s0; s < s1; ++s)
+    {
+        const z64* w = w2 + s * nspinor * npw2;
+        z64 u = w[g], d = nspinor == 2 ? w[npw2 + g] : z64{0, 0};
+        if (nspinor == 2) dm_su2(geo.su2, u, d);
+        u = cmul(u, f);
+        d = cmul(d, f);
+        if (!geo.tr2)
+        {
+            u.y = -u.y;
+            d.y = -d.y;
+        }
+        z64* o = wS2 + s * nspinor * npw1;
+        o[p] = u;
+        if (nspinor == 2) o[npw1 + p] = d;
+    }
 }
 
 // Batched complex FP64 GEMM for the q-star rotation (elph_q_rotate,

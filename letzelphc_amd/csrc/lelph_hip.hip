@@ -152,7 +152,7 @@ struct lelph_ctx
     DBuf cv_dv32;
     bool cv_dv32_valid = false;
     // electronic representation matrices
-    DBuf dm_map, dm_ph, dm_pos, dm_wRS, dm_wS2, dm_part, dm_out;
+    DBuf dm_map, dm_ph, dm_wRS, dm_wS2, dm_part, dm_out;
     // q-star rotation
     DBuf qr_dl, qr_dr, qr_g, qr_t, qr_out;
     // Fourier interpolation of dV_q
@@ -1066,7 +1066,7 @@ static void free_ctx(lelph_ctx* c)
                     &c->gbatch, &c->presplit,
                     &c->pl_cnt[0], &c->pl_cnt[1], &c->pl_off[0], &c->pl_off[1], &c->pl_cur[0],
                     &c->pl_cur[1], &c->pl_perm[0], &c->pl_perm[1], &c->dm_map, &c->dm_ph,
-                    &c->dm_pos, &c->dm_wRS, &c->dm_wS2, &c->dm_part, &c->dm_out, &c->qr_dl,
+                    &c->dm_wRS, &c->dm_wS2, &c->dm_part, &c->dm_out, &c->qr_dl,
                     &c->qr_dr, &c->qr_g, &c->qr_t, &c->qr_out, &c->ip_dvq, &c->ip_dvR,
                     &c->ip_last, &c->ip_tmp, &c->ip_out, &c->ip_ws, &c->ip_off, &c->ip_W,
                     &c->ip_P, &c->ip_qs, &c->ip_rot, &c->ip_eig, &c->lr_box, &c->lr_box2,
@@ -2636,23 +2636,22 @@ int lelph_electronic_reps(lelph_ctx* c, const double Rsym[9], const double tauR[
     const int nb = L.nbnds;
     LELPH_TRY(c->dm_map.ensure(sizeof(int) * c->nf));
     LELPH_TRY(c->dm_ph.ensure(sizeof(z64) * 3 * std::max<int64_t>(1, w1.npw)));
-    LELPH_TRY(c->dm_pos.ensure(sizeof(int) * std::max<int64_t>(1, w2.npw)));
     LELPH_TRY(c->dm_wRS.ensure(sizeof(z64) * nsets * Lk));
     LELPH_TRY(c->dm_wS2.ensure(sizeof(z64) * nsets * Lk));
-    HIP_TRY(hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream));
-    HIP_TRY(hipMemsetAsync(c->dm_map.p, 0xFF, sizeof(int) * c->nf, c->stream));
-    HIP_TRY(hipMemsetAsync(c->dm_wS2.p, 0, sizeof(z64) * nsets * Lk, c->stream));
+    // map to "no partner", wS2 (a missing partner contributes zero) and the
+    // error word cleared; then the first side; then both rotations
+    const int64_t most = std::max<int64_t>(c->nf, nsets * Lk);
+    hipLaunchKernelGGL(k_dm_clear, dim3((unsigned)std::min<int64_t>(cdiv(most, 256), 4096)),
+                       dim3(256), 0, c->stream, c->dm_map.as<int>(), c->nf, c->dm_wS2.as<z64>(),
+                       nsets * Lk, c->d_err);
     hipLaunchKernelGGL(k_dm_side1, dim3((unsigned)cdiv(w1.npw, 256)), dim3(256), 0, c->stream,
                        w1.gvec, w1.npw, geo, Nx, Ny, Nz, c->dm_map.as<int>(), c->dm_ph.as<z64>(),
                        c->d_err);
-    hipLaunchKernelGGL(k_dm_side2, dim3((unsigned)cdiv(w2.npw, 256)), dim3(256), 0, c->stream,
-                       w2.gvec, w2.npw, geo, Nx, Ny, Nz, c->dm_map.as<int>(), c->dm_pos.as<int>());
-    hipLaunchKernelGGL(k_dm_rot1, dim3((unsigned)cdiv(nsets * w1.npw, 256)), dim3(256), 0,
-                       c->stream, w1.wfc, nsets, L.nspinor, w1.npw, c->dm_ph.as<z64>(), geo,
-                       c->dm_wRS.as<z64>());
-    hipLaunchKernelGGL(k_dm_rot2, dim3((unsigned)cdiv(nsets * w2.npw, 256)), dim3(256), 0,
-                       c->stream, w2.wfc, nsets, L.nspinor, w2.npw, w1.npw, c->dm_pos.as<int>(),
-                       c->dm_ph.as<z64>(), geo, c->dm_wS2.as<z64>());
+    const int64_t gb = std::max(w1.npw, w2.npw);
+    hipLaunchKernelGGL(k_dm_rot, dim3((unsigned)cdiv(gb, 128), (unsigned)cdiv(nsets, DM_SETS), 2),
+                       dim3(128), 0, c->stream, w1.wfc, w1.npw, w2.gvec, w2.wfc, w2.npw, nsets,
+                       L.nspinor, geo, Nx, Ny, Nz, c->dm_map.as<int>(), c->dm_ph.as<z64>(),
+                       c->dm_wRS.as<z64>(), c->dm_wS2.as<z64>());
     HIP_TRY(hipGetLastError());
     // D[s] = wS2[s] (nb x Lk) . wRS[s]^T (:377-394), split over the sphere
     const int64_t nchunks = cdiv(Lk, CT_KC);
