@@ -83,6 +83,7 @@ struct DBuf
 } // namespace
 
 #include "convpath_bufs.hpp"
+#include "copyout.hpp"
 
 struct lelph_ctx
 {
@@ -181,6 +182,7 @@ struct lelph_ctx
     // device time of the last lelph_interp_dvscf: weights, R -> q, long range, total, nq
     hipEvent_t ip_ev[4] = {nullptr, nullptr, nullptr, nullptr};
     double ip_ms[5] = {0, 0, 0, 0, 0};
+    CopyOut copy_out;
     NlBufs nl; // non-local part
     std::vector<NlWindow> nl_win; // of the batch under way
     int64_t nl_step = 1;          // pairs of one window
@@ -1060,6 +1062,7 @@ static void free_ctx(lelph_ctx* c)
         if (p) (void)hipFree(p);
     c->cv.release();
     c->nl.release();
+    c->copy_out.release();
     c->cv_dv32.release();
     DBuf* bufs[] = {&c->dv64, &c->dv32, &c->eig_d, &c->vloc_tmp, &c->rot_tmp, &c->idx_k,
                     &c->idx_kq, &c->ph_k, &c->ph_kq, &c->box_k, &c->box_kq, &c->box_x, &c->part, &c->g,
@@ -3167,6 +3170,8 @@ int lelph_interp_finish(lelph_ctx* c)
                        dim3(256), 0, c->stream, c->ip_P.as<z64>(), (int)nq, (int)nq, 1,
                        c->ip_dvq.as<z64>(), 1, cols, c->ip_dvR.as<z64>(), nullptr, 0, 0, 0);
     HIP_TRY(hipGetLastError());
+    // the results' staging, beside the transform (without it: plain copies)
+    if (sizeof(z64) * (size_t)cols >= COPY_OUT_CHUNK / 2) (void)c->copy_out.ensure();
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->ip_dvq.release();
     c->ip_ready = true;
@@ -3229,9 +3234,8 @@ int lelph_interp_dvscf(lelph_ctx* c, int64_t nq, const double* qpts, double* dvs
     {
         const int64_t n = std::min(chunk, nq - q0);
         LELPH_TRY(ip_r2q(c, n, qpts + 3 * q0, c->ip_out.as<z64>()));
-        HIP_TRY(hipMemcpyAsync(reinterpret_cast<char*>(dvscf_out) + per * q0, c->ip_out.p,
-                               per * n, hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(hipStreamSynchronize(c->stream));
+        LELPH_TRY(c->copy_out.run(reinterpret_cast<char*>(dvscf_out) + per * q0, c->ip_out.p,
+                                  per * n, c->stream));
     }
     return check_err(c);
 }

@@ -214,11 +214,13 @@ static int nl_modes(lelph_ctx* c, const z64* ebuf, int64_t n, z64* g, hipStream_
     const lelph_lattice& L = c->lat;
     const int64_t es = (int64_t)L.nspin * L.nbnds * L.nbnds;
     const z64 pre = {0.0, -2 * LELPH_RPI * LELPH_E2};
-    hipLaunchKernelGGL(k_nl_mode,
-                       dim3((unsigned)cdiv(es, 256), (unsigned)cdiv(L.nmodes, NL_MODES),
-                            (unsigned)n),
-                       dim3(256), 0, st, ebuf, c->eig_d.as<z64>(), L.nmodes,
-                       3 * L.natom, es, pre, g);
+    const int64_t one = nl_sum_size(c), gsz = (int64_t)L.nmodes * es;
+    for (int64_t p = 0; p < n; p += 32768) // grid limit
+        hipLaunchKernelGGL(k_nl_mode,
+                           dim3((unsigned)cdiv(es, 256), (unsigned)cdiv(L.nmodes, NL_MODES),
+                                (unsigned)std::min<int64_t>(32768, n - p)),
+                           dim3(256), 0, st, ebuf + p * one, c->eig_d.as<z64>(), L.nmodes,
+                           3 * L.natom, es, pre, g + p * gsz);
     HIP_TRY(hipGetLastError());
     return LELPH_OK;
 }
