@@ -147,7 +147,10 @@ int lelph_set_precision(lelph_ctx* ctx, int precision);
  * by the project's autotuner (letzelphc_amd/autotune.py).  fft_lines and
  * fp32_form give bit-identical g; split_target moves the boundaries of the
  * fixed-order FP64 sum (g changes at the rounding level).  Zero fields
- * take the defaults. */
+ * take the defaults.  split_target, fft_lines, fp32_form and ctile act where
+ * the local part is contracted over the whole box; where it is transformed to
+ * the k+q sphere instead (chosen from sizes and precision) they change
+ * nothing. */
 typedef struct lelph_tuning
 {
     int split_target; /* blocks aimed at by the FP64/FP32 contraction's K
