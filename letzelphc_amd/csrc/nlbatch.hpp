@@ -28,10 +28,11 @@ struct NlKey
 };
 
 // Rotated psi (blockIdx.y < ngy: sets in groups of spy) and projectors
-// (blockIdx.y - ngy = a * pmax + p: beta[(a*pmax + p)*4 + x][G], F_l(K)
-// e^{-2 pi i K.tau_a} Y_lm(K) and K-weighted) of one side (blockIdx.z).  K and
-// Y_lm are recomputed where they are used: the tables of them cost a launch
-// between the two.
+// (blockIdx.y - ngy: NL_PROJ of an atom, beta[(a*pmax + p)*4 + x][G] = F_l(K)
+// e^{-2 pi i K.tau_a} Y_lm(K), and K-weighted) of one side (blockIdx.z).  The
+// phase and the direction of K are formed once per thread (with one projector
+// per thread they were most of its time); tables of them would cost a launch.
+#define NL_PROJ 4
 template <typename T>
 __global__ __launch_bounds__(128) void k_nl_sides(
     const NlKey* __restrict__ keys, int64_t nsets, int nspinor, int spy, int ngy, NlProj pj,
@@ -74,26 +75,33 @@ __global__ __launch_bounds__(128) void k_nl_sides(
         }
         return;
     }
-    const int ap = blockIdx.y - ngy, a = ap / pj.pmax;
-    const int* e = plist + 3 * ap;
-    const auto b = gptr<T>::of(k.beta) + (int64_t)ap * 4 * npw;
-    if (e[0] < 0)
-    {
-        for (int x = 0; x < 4; ++x) b.set((int64_t)x * npw + g, {0, 0});
-        return;
-    }
-    const int lidx = e[0], l = e[1], ty = atype[a];
+    const int npg = (pj.pmax + NL_PROJ - 1) / NL_PROJ, yb = blockIdx.y - ngy, a = yb / npg;
+    const int p0 = (yb % npg) * NL_PROJ, p1 = min(p0 + NL_PROJ, pj.pmax);
+    const int ty = atype[a];
     const double* tau = apos + 3 * a;
     sincos(-2.0 * LELPH_RPI * (K[0] * tau[0] + K[1] * tau[1] + K[2] * tau[2]), &s, &c);
-    const double f =
-        g_of(k.Fk)[((int64_t)lidx * pj.ntype + ty) * npw + g] * d_Ylm(l, e[2] - l * l - l, K);
-    const z64 b0 = {f * c, f * s};
-    const double sg = Fsign[lidx * pj.ntype + ty];
-    b.set(g, {(T)b0.x, (T)b0.y});
-    for (int x = 0; x < 3; ++x)
+    const YlmDir dir(K);
+    for (int p = p0; p < p1; ++p)
     {
-        const double kx = K[x] * sg;
-        b.set((int64_t)(x + 1) * npw + g, {(T)(b0.x * kx), (T)(b0.y * kx)});
+        const int ap = a * pj.pmax + p;
+        const int* e = plist + 3 * ap;
+        const auto b = gptr<T>::of(k.beta) + (int64_t)ap * 4 * npw;
+        if (e[0] < 0)
+        {
+            for (int x = 0; x < 4; ++x) b.set((int64_t)x * npw + g, {0, 0});
+            continue;
+        }
+        const int lidx = e[0], l = e[1];
+        const double f =
+            g_of(k.Fk)[((int64_t)lidx * pj.ntype + ty) * npw + g] * d_Ylm(l, e[2] - l * l - l, dir);
+        const z64 b0 = {f * c, f * s};
+        const double sg = Fsign[lidx * pj.ntype + ty];
+        b.set(g, {(T)b0.x, (T)b0.y});
+        for (int x = 0; x < 3; ++x)
+        {
+            const double kx = K[x] * sg;
+            b.set((int64_t)(x + 1) * npw + g, {(T)(b0.x * kx), (T)(b0.y * kx)});
+        }
     }
 }
 

@@ -153,7 +153,8 @@ static int nl_sides_t(lelph_ctx* c, NlBufs& b, DBuf& desc, const NlWindow& w, bo
         }
         const NlKey* dk = desc.as<NlKey>() + k0;
         hipLaunchKernelGGL(k_nl_sides<T>,
-                           dim3((unsigned)cdiv(npw, 128), ngy + L.natom * c->pmax, (unsigned)n),
+                           dim3((unsigned)cdiv(npw, 128), ngy + L.natom * (unsigned)cdiv(c->pmax, NL_PROJ),
+                                (unsigned)n),
                            dim3(128), 0, st, dk, nsb, L.nspinor, NL_SPY, (int)ngy, pj, c->d_plist,
                            c->d_atype, c->d_apos, c->d_Fsign);
         HIP_TRY(hipGetLastError());

@@ -47,13 +47,24 @@ __device__ inline double d_legendre(int l, int m, double x)
     return p;
 }
 
-// Ylm (src/common/numerical_func.c:97-152): real harmonics, Blanco et al.
-__device__ inline double d_Ylm(int l, int m, const double* v)
+// Ylm (src/common/numerical_func.c:97-152): real harmonics, Blanco et al.;
+// the direction once, then any number of (l, m)
+struct YlmDir
 {
-    const double nrm = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-    if (nrm < LELPH_EPS6) return l != 0 ? 0.0 : 1.0 / sqrt(4 * LELPH_RPI);
-    const double cost = v[2] / nrm;
-    const double phi = atan2(v[1], v[0]);
+    double cost, phi;
+    bool zero;
+    __device__ explicit YlmDir(const double* v)
+    {
+        const double nrm = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+        zero = nrm < LELPH_EPS6;
+        cost = zero ? 0.0 : v[2] / nrm;
+        phi = zero ? 0.0 : atan2(v[1], v[0]);
+    }
+};
+__device__ inline double d_Ylm(int l, int m, const YlmDir& dir)
+{
+    if (dir.zero) return l != 0 ? 0.0 : 1.0 / sqrt(4 * LELPH_RPI);
+    const double cost = dir.cost, phi = dir.phi;
     double sh;
     if (m > 0)
         sh = sqrt(2.0) * cos(m * phi);
