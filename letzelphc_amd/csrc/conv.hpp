@@ -536,8 +536,8 @@ struct ConvSrc
 };
 
 // FP64 lines exchange their real and imaginary parts one after the other
-// through the same rows: half the LDS, so that 12 waves and not 8 share a CU
-// beside a 96 x 96 plane buffer.
+// through the same rows: half the LDS, so that the rows of 8 waves (41 KB) fit
+// beside a 96 x 96 plane buffer (80 KB) and its tables.
 template <typename T>
 constexpr bool ln_split()
 {
