@@ -185,6 +185,72 @@ static int conv_ensure_dv32(lelph_ctx* c, const ConvGeo& g)
     return LELPH_OK;
 }
 
+// bytes of a group's buffers and of their parts: np pairs, ns sides (a k+q
+// one per pair, the distinct k ones)
+struct ConvLayout
+{
+    size_t n_mask, o_ph, s_ph, s_idx, s_smap, s_zc, s_off, per; // maps of a side
+    size_t s_coef, s_line, s_box;                               // of a side
+    size_t s_cl, s_c;                                           // of a pair
+    size_t map, coef, line, box, c, part;
+    static size_t up(size_t n) { return (n + 255) & ~(size_t)255; }
+    ConvLayout(const lelph_ctx* ctx, const ConvGeo& g, const ConvGroup& gr, int np, int ns)
+    {
+        const lelph_lattice& L = ctx->lat;
+        const size_t Nx = (size_t)L.fft_dims[0], Ny = (size_t)L.fft_dims[1];
+        const size_t Nz = (size_t)L.fft_dims[2], item = g.f32 ? sizeof(c32) : sizeof(z64);
+        n_mask = up(4 * Ny * Nz * g.words);
+        o_ph = up(n_mask * (size_t)ns);
+        s_ph = up(sizeof(z64) * g.npw);
+        s_idx = up(4 * (size_t)g.npw);
+        s_smap = up(4 * (size_t)g.nzk * Ny);
+        s_zc = up(2 * Nz);
+        s_off = up(4 * (size_t)g.nst);
+        per = s_ph + s_idx + s_smap + s_zc + s_off + up(4 * (size_t)g.nst * g.words) + 256;
+        const size_t row = item * (size_t)g.nrows;
+        s_coef = row * g.ld;
+        s_line = row * Nx * g.nst;
+        s_box = row * (size_t)ctx->nf;
+        s_cl = item * (size_t)gr.ns * gr.nv * Nx * g.nst;
+        s_c = s_coef * L.nmodes;
+        map = o_ph + per * ns;
+        coef = s_coef * ns;
+        line = std::max(s_line * (ns - np), s_cl * np);
+        box = s_box * (ns - np);
+        c = s_c * np;
+        const size_t gsz = (size_t)L.nmodes * L.nspin * L.nbnds * L.nbnds;
+        part = g.nsplit > 1 ? sizeof(z64) * (size_t)g.nsplit * np * gsz : 0;
+    }
+    int ensure(ConvBufs& b, hipStream_t st) const
+    {
+        LELPH_TRY(buf_grow(b.map, map, b.fixed, st));
+        LELPH_TRY(buf_grow(b.coef, coef, b.fixed, st));
+        LELPH_TRY(buf_grow(b.line, line, b.fixed, st));
+        LELPH_TRY(buf_grow(b.box, box, b.fixed, st));
+        LELPH_TRY(buf_grow(b.c, c, b.fixed, st));
+        return buf_grow(b.part, part, b.fixed, st);
+    }
+};
+
+// Sizes b for every group of these pairs, for good: their descriptors, which
+// hold its addresses, are run again by a captured pass.
+static int conv_reserve(lelph_ctx* c, const ConvGeo& g, const ConvGroup& gr, ConvBufs& b,
+                        const std::vector<lelph_pair>& pairs, hipStream_t st)
+{
+    for (size_t p0 = 0; p0 < pairs.size(); p0 += gr.np)
+    {
+        const size_t p1 = std::min(pairs.size(), p0 + gr.np);
+        std::vector<std::array<int, 2>> k;
+        for (size_t i = p0; i < p1; ++i) k.push_back({pairs[i].ik, pairs[i].ksym});
+        std::sort(k.begin(), k.end());
+        const int nk = (int)(std::unique(k.begin(), k.end()) - k.begin());
+        const int np = (int)(p1 - p0);
+        LELPH_TRY(ConvLayout(c, g, gr, np, np + nk).ensure(b, st));
+    }
+    b.fixed = true;
+    return LELPH_OK;
+}
+
 // local part of `np` pairs into g (device, np * gsz contiguous) on stream
 // st.  ev: [1] boxes built, [2] products done, or NULL.  desc: the group's
 // descriptors, uploaded unless they are there already (a captured pass).
@@ -233,52 +299,36 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
         kside[i] = at;
     }
     const int ns = (int)sides.size(), nk = ns - np;
-    // map arena of a side
-    const size_t cells = (size_t)Ny * Nz;
-    auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
-    const size_t o_mask = 0, n_mask = up(4 * cells * geo.words);
-    const size_t o_ph = up(n_mask * (size_t)ns);
-    const size_t s_ph = up(sizeof(z64) * geo.npw), s_idx = up(4 * (size_t)geo.npw);
-    const size_t s_smap = up(4 * (size_t)geo.nzk * Ny), s_zc = up(2 * (size_t)Nz);
-    const size_t s_off = up(4 * (size_t)geo.nst), s_sm = up(4 * (size_t)geo.nst * geo.words);
-    const size_t per = s_ph + s_idx + s_smap + s_zc + s_off + s_sm + 256;
-    LELPH_TRY(b.map.ensure(o_ph + per * ns));
-    const size_t row = sizeof(cpx<T>) * (size_t)geo.nrows;
-    const size_t s_coef = row * geo.ld, s_line = row * Nx * geo.nst, s_box = row * c->nf;
-    LELPH_TRY(b.coef.ensure(s_coef * ns));
-    const size_t s_cl = sizeof(cpx<T>) * (size_t)nset * nv * Nx * geo.nst, s_c = s_coef * L.nmodes;
-    LELPH_TRY(b.line.ensure(std::max(s_line * nk, s_cl * np)));
-    LELPH_TRY(b.box.ensure(s_box * nk));
-    LELPH_TRY(b.c.ensure(s_c * np));
+    const ConvLayout lay(c, geo, gr, np, ns);
+    LELPH_TRY(lay.ensure(b, st));
     const int64_t gsz = (int64_t)L.nmodes * L.nspin * L.nbnds * L.nbnds;
-    if (geo.nsplit > 1) LELPH_TRY(b.part.ensure(sizeof(z64) * (size_t)geo.nsplit * np * gsz));
     char* m0 = b.map.as<char>();
     for (int i = 0; i < ns; ++i)
     {
         SphSide& s = sides[i];
         s.ld = (int)(cdiv(s.npw, 16) * 16);
-        s.mask = reinterpret_cast<unsigned*>(m0 + o_mask + n_mask * i);
-        char* m = m0 + o_ph + per * i;
+        s.mask = reinterpret_cast<unsigned*>(m0 + lay.n_mask * i);
+        char* m = m0 + lay.o_ph + lay.per * i;
+        s.cnt = reinterpret_cast<int*>(m + lay.per - 256);
         s.ph = reinterpret_cast<z64*>(m);
-        s.idx = reinterpret_cast<int*>(m += s_ph);
-        s.smap = reinterpret_cast<int*>(m += s_idx);
-        s.zc = reinterpret_cast<short*>(m += s_smap);
-        s.off = reinterpret_cast<int*>(m += s_zc);
-        s.smask = reinterpret_cast<unsigned*>(m += s_off);
-        s.cnt = reinterpret_cast<int*>(m += s_sm);
-        s.coef = b.coef.as<char>() + s_coef * i;
-        s.line = i < np ? nullptr : b.line.as<char>() + s_line * (i - np);
-        s.box = i < np ? nullptr : b.box.as<char>() + s_box * (i - np);
+        s.idx = reinterpret_cast<int*>(m += lay.s_ph);
+        s.smap = reinterpret_cast<int*>(m += lay.s_idx);
+        s.zc = reinterpret_cast<short*>(m += lay.s_smap);
+        s.off = reinterpret_cast<int*>(m += lay.s_zc);
+        s.smask = reinterpret_cast<unsigned*>(m += lay.s_off);
+        s.coef = b.coef.as<char>() + lay.s_coef * i;
+        s.line = i < np ? nullptr : b.line.as<char>() + lay.s_line * (i - np);
+        s.box = i < np ? nullptr : b.box.as<char>() + lay.s_box * (i - np);
     }
     for (int i = 0; i < np; ++i)
     {
         cp[i].box = sides[kside[i]].box;
         cp[i].dv = geo.f32 ? c->cv_dv32.p : c->dv64.p;
         cp[i].side = i;
-        cp[i].line = b.line.as<char>() + s_cl * i;
-        cp[i].c = b.c.as<char>() + s_c * i;
+        cp[i].line = b.line.as<char>() + lay.s_cl * i;
+        cp[i].c = b.c.as<char>() + lay.s_c * i;
     }
-    const size_t n_s = up(sizeof(SphSide) * ns);
+    const size_t n_s = ConvLayout::up(sizeof(SphSide) * ns);
     std::vector<char> hd(n_s + sizeof(ConvPair) * np);
     std::memcpy(hd.data(), sides.data(), sizeof(SphSide) * ns);
     std::memcpy(hd.data() + n_s, cp.data(), sizeof(ConvPair) * np);
@@ -292,7 +342,7 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
     const z64 *Wx = axis_tw<double>(c->ax[0]), *Wy = axis_tw<double>(c->ax[1]),
               *Wz = axis_tw<double>(c->ax[2]);
 
-    LELPH_TRY(zero_async(m0 + o_mask, n_mask * ns, st));
+    LELPH_TRY(zero_async(m0, lay.n_mask * ns, st));
     LELPH_TRY(conv_maps_launch(ns, geo.npw, st, ds, Nx, Ny, Nz, geo.words, geo.nzk, geo.nst,
                                c->d_err));
     const int64_t nsets = (int64_t)L.nspin * L.nbnds;

@@ -3,10 +3,22 @@
 // Included by lelph_hip.hip before the context, which owns a set.
 #pragma once
 
+// Grows b to need bytes; work on st that may still use it ends first.  fixed:
+// uploaded descriptors that are run again (a captured pass) hold b's address,
+// so it must be large enough already.
+static int buf_grow(DBuf& b, size_t need, bool fixed, hipStream_t st)
+{
+    if (need <= b.n) return LELPH_OK;
+    if (fixed) return LELPH_ERR_STATE;
+    if (b.p) HIP_TRY(hipStreamSynchronize(st));
+    return b.ensure(need);
+}
+
 // working buffers of one stream of groups
 struct ConvBufs
 {
     DBuf desc, map, coef, line, box, c, part;
+    bool fixed = false; // sized for every group that uses them (conv_reserve)
     void release()
     {
         for (DBuf* b : {&desc, &map, &coef, &line, &box, &c, &part}) b->release();
@@ -18,6 +30,7 @@ struct ConvBufs
 struct NlBufs
 {
     DBuf desc, side, bb, ebuf, splitA, splitB;
+    bool fixed = false; // sized for every window that uses them (nl_reserve)
     const int* kk = nullptr; // pairs' key numbers of the current window
     void release()
     {

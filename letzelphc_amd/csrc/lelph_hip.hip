@@ -1958,8 +1958,9 @@ struct lelph_multi
     std::vector<MultiPair> pairs;
     std::vector<int64_t> border; // box build order: each cell's pairs along chains
     int non_loc = 1;
-    // cells in the sphere form: their buffers and, per group of pairs, the
-    // descriptors that the captured pass reads
+    // cells in the sphere form: their buffers, sized for every group before
+    // the first one runs, and, per group of pairs, the descriptors that the
+    // captured pass reads
     struct ConvCell
     {
         bool on = false;
@@ -1970,8 +1971,8 @@ struct lelph_multi
         std::vector<lelph_pair> pairs;
     };
     std::vector<ConvCell> conv;
-    // non-local parts: per cell its buffers (the sums of all its pairs) and
-    // per window of pairs the sides and their descriptors
+    // non-local parts: per cell its buffers (sized for every window; the sums
+    // of all its pairs) and per window of pairs the sides and their descriptors
     struct NlCell
     {
         NlBufs bufs;
@@ -2348,6 +2349,8 @@ static int multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
             cc.pairs.assign(pairs[i], pairs[i] + npairs[i]);
             cc.desc.resize((size_t)cdiv(npairs[i], cc.gr.np));
             int st = conv_prepare(c, cc.geo);
+            if (st == LELPH_OK)
+                st = conv_reserve(c, cc.geo, cc.gr, cc.bufs, cc.pairs, m->stream);
             if (st != LELPH_OK) return fail(st);
         }
         else if (prec == LELPH_FP32)
@@ -2366,6 +2369,8 @@ static int multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
                 nc.win.back().add(pairs[i][j]);
             }
             nc.desc.resize(nc.win.size());
+            int st = nl_reserve(c, nc.bufs, nc.win, m->nl);
+            if (st != LELPH_OK) return fail(st);
             if (nc.bufs.ebuf.ensure(sizeof(z64) * (size_t)(nl_sum_size(c) * npairs[i])))
                 return fail(LELPH_ERR_ALLOC);
         }

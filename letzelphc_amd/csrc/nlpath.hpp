@@ -32,13 +32,6 @@ struct NlDims
     }
 };
 
-// a buffer that work on st may still use grows once that work is done
-static int nl_ensure(DBuf& b, size_t need, hipStream_t st)
-{
-    if (need > b.n && b.p) HIP_TRY(hipStreamSynchronize(st));
-    return b.ensure(need);
-}
-
 // pairs per window: of `step` pairs at a time
 static int64_t nl_window(const lelph_ctx* c, int64_t step, int64_t npairs)
 {
@@ -70,6 +63,72 @@ static int nl_gemm_split(NlBufs& b, const z64* A, const z64* B, int rows, int64_
     return reduce_parts(part, nsplit, (int64_t)rows * ncol, 1.0, out, st);
 }
 
+static int nl_check(const lelph_ctx* c, const NlWindow& w)
+{
+    for (const auto& k : w.keys)
+        if (!c->wf[k[0]].wfc || !c->wf[k[0]].Fk) return LELPH_ERR_STATE;
+    return LELPH_OK;
+}
+
+// the GEMM splits of a window's sides and the bytes it takes
+struct NlLayout
+{
+    std::vector<int64_t> cps;
+    std::vector<int> nsplit;
+    size_t side_max = 0; // scratch of a side
+    int per = 1;         // sides formed together
+    size_t side = 0, bb = 0, splitA = 0, splitB = 0;
+    NlLayout(const lelph_ctx* c, const NlDims& d, const NlWindow& w)
+    {
+        const size_t nk = w.keys.size(), item = d.f32 ? sizeof(c32) : sizeof(z64);
+        const int64_t count = d.rows * d.ncol;
+        const int64_t tiles = cdiv(d.rows, GZ_MB) * cdiv(d.ncol, GZ_NB);
+        int64_t npw_max = 0;
+        cps.resize(nk);
+        nsplit.resize(nk);
+        for (size_t i = 0; i < nk; ++i)
+        {
+            const int64_t npw = c->wf[w.keys[i][0]].npw;
+            pick_splits(tiles, cdiv(npw, d.split ? 32 : CT_KC), count, &cps[i], &nsplit[i]);
+            npw_max = std::max(npw_max, npw);
+            const size_t one = item * (size_t)npw * (d.ncol + d.rows) +
+                               sizeof(z64) * (size_t)(nsplit[i] * count) + 64;
+            side_max = std::max(side_max, (one + 255) & ~(size_t)255);
+        }
+        per = (int)std::max<size_t>(1, std::min<size_t>(nk, NL_SCRATCH_BYTES / side_max));
+        side = side_max * per;
+        bb = sizeof(z64) * nk * (size_t)count;
+        if (d.split)
+        {
+            const int64_t Kp = cdiv(npw_max, 32) * 32;
+            splitA = sizeof(__bf16) * 6 * (size_t)(cdiv(d.rows, 64) * 64 * Kp);
+            splitB = sizeof(__bf16) * 6 * (size_t)(cdiv(d.ncol, 64) * 64 * Kp);
+        }
+    }
+    int ensure(NlBufs& b, hipStream_t st) const
+    {
+        LELPH_TRY(buf_grow(b.side, side, b.fixed, st));
+        LELPH_TRY(buf_grow(b.bb, bb, b.fixed, st));
+        LELPH_TRY(buf_grow(b.splitA, splitA, b.fixed, st));
+        return buf_grow(b.splitB, splitB, b.fixed, st);
+    }
+};
+
+// Sizes b for all of these windows, for good: their descriptors, which hold
+// its addresses, are run again by a captured pass.
+static int nl_reserve(const lelph_ctx* c, NlBufs& b, const std::vector<NlWindow>& win,
+                      hipStream_t st)
+{
+    const NlDims d(c);
+    for (const NlWindow& w : win)
+    {
+        LELPH_TRY(nl_check(c, w));
+        LELPH_TRY(NlLayout(c, d, w).ensure(b, st));
+    }
+    b.fixed = true;
+    return LELPH_OK;
+}
+
 // <beta_K|psi> of the window's sides into b.bb on stream st.  upload: the
 // descriptors are copied over (a captured pass finds them there).  Nothing
 // of an earlier window may still run on another stream than st.
@@ -81,14 +140,14 @@ static int nl_sides_t(lelph_ctx* c, NlBufs& b, DBuf& desc, const NlWindow& w, bo
     const NlDims d(c);
     const int64_t nsb = (int64_t)L.nspin * L.nbnds, count = d.rows * d.ncol;
     const int nk = (int)w.keys.size();
-    // sizes of a side and of the sides formed together
-    size_t side_max = 0;
-    int64_t npw_max = 0;
+    LELPH_TRY(nl_check(c, w));
+    const NlLayout lay(c, d, w);
+    const size_t side_max = lay.side_max;
+    const int per = lay.per;
     std::vector<NlKey> hk((size_t)nk);
     for (int i = 0; i < nk; ++i)
     {
         const DevWfc& v = c->wf[w.keys[i][0]];
-        if (!v.wfc || !v.Fk) return LELPH_ERR_STATE;
         const lelph_symmetry& S = c->syms[w.keys[i][1]];
         NlKey& k = hk[i];
         k = NlKey{};
@@ -96,28 +155,15 @@ static int nl_sides_t(lelph_ctx* c, NlBufs& b, DBuf& desc, const NlWindow& w, bo
         k.wfc = v.wfc;
         k.Fk = v.Fk;
         k.npw = v.npw;
+        k.cps = lay.cps[i];
+        k.nsplit = lay.nsplit[i];
         std::memcpy(k.sd.S, S.Rmat, sizeof(k.sd.S));
         std::memcpy(k.sd.k, c->kpt_ibz.data() + 3 * w.keys[i][0], sizeof(k.sd.k));
         std::memcpy(k.sd.tau, S.tau, sizeof(k.sd.tau));
         k.sd.conj_w = S.time_rev ? 0 : 1; // 'C' unless time reversed (Vbare_nloc.c:397-407)
         LELPH_TRY(su2mat(S.Rmat, L.nspinor, S.time_rev, k.sd.su2));
-        const int64_t nch = cdiv(v.npw, d.split ? 32 : CT_KC);
-        const int64_t tiles = cdiv(d.rows, GZ_MB) * cdiv(d.ncol, GZ_NB);
-        pick_splits(tiles, nch, count, &k.cps, &k.nsplit);
-        npw_max = std::max(npw_max, v.npw);
-        const size_t one = sizeof(cpx<T>) * (size_t)v.npw * (d.ncol + d.rows) +
-                           sizeof(z64) * (size_t)(k.nsplit * count) + 64;
-        side_max = std::max(side_max, (one + 255) & ~(size_t)255);
     }
-    const int per = (int)std::max<size_t>(1, std::min<size_t>((size_t)nk, NL_SCRATCH_BYTES / side_max));
-    LELPH_TRY(nl_ensure(b.side, side_max * per, st));
-    LELPH_TRY(nl_ensure(b.bb, sizeof(z64) * (size_t)(nk * count), st));
-    if (d.split)
-    {
-        const int64_t Kp = cdiv(npw_max, 32) * 32;
-        LELPH_TRY(nl_ensure(b.splitA, sizeof(__bf16) * 6 * (size_t)(cdiv(d.rows, 64) * 64 * Kp), st));
-        LELPH_TRY(nl_ensure(b.splitB, sizeof(__bf16) * 6 * (size_t)(cdiv(d.ncol, 64) * 64 * Kp), st));
-    }
+    LELPH_TRY(lay.ensure(b, st));
     for (int i = 0; i < nk; ++i)
     {
         NlKey& k = hk[i];
@@ -132,7 +178,7 @@ static int nl_sides_t(lelph_ctx* c, NlBufs& b, DBuf& desc, const NlWindow& w, bo
     const size_t nb_k = sizeof(NlKey) * (size_t)nk, nb_kk = sizeof(int) * w.kk.size();
     if (upload)
     {
-        LELPH_TRY(nl_ensure(desc, nb_k + nb_kk, st));
+        LELPH_TRY(buf_grow(desc, nb_k + nb_kk, false, st));
         std::vector<char> host(nb_k + nb_kk);
         std::memcpy(host.data(), hk.data(), nb_k);
         std::memcpy(host.data() + nb_k, w.kk.data(), nb_kk);
@@ -232,7 +278,7 @@ static int nl_modes(lelph_ctx* c, const z64* ebuf, int64_t n, z64* g, hipStream_
 static int nl_add(lelph_ctx* c, NlBufs& b, int64_t p0, int64_t n, z64* g, hipStream_t st,
                   hipEvent_t after)
 {
-    LELPH_TRY(nl_ensure(b.ebuf, sizeof(z64) * (size_t)(nl_sum_size(c) * n), st));
+    LELPH_TRY(buf_grow(b.ebuf, sizeof(z64) * (size_t)(nl_sum_size(c) * n), false, st));
     LELPH_TRY(nl_sums(c, b, p0, n, b.ebuf.as<z64>(), st));
     if (after) HIP_TRY(hipStreamWaitEvent(st, after, 0));
     return nl_modes(c, b.ebuf.as<z64>(), n, g, st);
