@@ -149,8 +149,7 @@ int lelph_set_precision(lelph_ctx* ctx, int precision);
  * fixed-order FP64 sum (g changes at the rounding level).  Zero fields
  * take the defaults.  split_target, fft_lines, fp32_form and ctile act where
  * the local part is contracted over the whole box; where it is transformed to
- * the k+q sphere instead (chosen from sizes and precision) they change
- * nothing. */
+ * the k+q sphere instead (lelph_set_local_form) they change nothing. */
 typedef struct lelph_tuning
 {
     int split_target; /* blocks aimed at by the FP64/FP32 contraction's K
@@ -170,6 +169,24 @@ typedef struct lelph_tuning
 } lelph_tuning;
 int lelph_set_tuning(lelph_ctx* ctx, const lelph_tuning* tuning);
 int lelph_get_tuning(lelph_ctx* ctx, lelph_tuning* tuning);
+
+/* The form of the local part: contracted over the whole box
+ * (LELPH_FORM_BOX), or transformed to the k+q sphere and contracted there
+ * (LELPH_FORM_SPHERE).  LELPH_FORM_AUTO, the default, takes the one that is
+ * faster at the context's sizes and precision; LELPH_FORM_SPHERE takes the
+ * sphere form wherever it applies (axis lengths it is compiled for, planes
+ * that fit in LDS, no two plane waves of a sphere on one box point).
+ * lelph_get_local_form: the form asked for and the one that the context's
+ * calls take as it stands (BOX or SPHERE); either pointer may be NULL.  No
+ * counterpart in the reference. */
+enum
+{
+    LELPH_FORM_AUTO = 0,
+    LELPH_FORM_BOX = 1,
+    LELPH_FORM_SPHERE = 2
+};
+int lelph_set_local_form(lelph_ctx* ctx, int form);
+int lelph_get_local_form(lelph_ctx* ctx, int* requested, int* used);
 
 /* The precision requested with lelph_create / lelph_set_precision and the
  * one the contractions run in on this context's shape: LELPH_BF16X3 runs as

@@ -23,6 +23,7 @@ STATUS_NAMES = {
 }
 
 PRECISIONS = {"fp64": 0, "fp32": 1, "bf16x3": 2, "bf16x6": 3}
+LOCAL_FORMS = {"auto": 0, "box": 1, "sphere": 2}
 KERNELS = {"dfpt": 0, "dfpt_local": 1, "bare": 2, "bare_local": 3}
 
 

@@ -25,7 +25,9 @@ each candidate timed on a few pairs of the actual workload with the
 library's own HIP-event timings (lelph_last_timings, device time of the
 batch), the median of `reps` runs, and checked against the g of the
 shape it departs from.  Results go to a JSON cache
-(LELPH_TUNE_CACHE, default letzelphc_amd/tune_cache.json).
+(LELPH_TUNE_CACHE, default letzelphc_amd/tune_cache.json).  All knobs belong
+to the box form of the local part (lelph_set_local_form): a context in the
+sphere form is timed once, with the defaults, and not cached.
 """
 from __future__ import annotations
 
@@ -106,6 +108,9 @@ def tune(ctx, pairs, qpt, sample: int = 3, reps: int = 3, cache: dict | None = N
     best = {"split_target": 0, "fft_lines": 0, "fp32_form": 0, "ctile": 0}
     ctx.set_tuning(**best)
     base_ms, ref = _time(ctx, sub, qpt, reps)
+    if ctx.local_form() != "box":
+        return {"tuning": best, "ms": base_ms, "default_ms": base_ms, "tried": 1,
+                "pairs_timed": len(sub), "cached": False}
     best_ms, best_g = base_ms, ref
     tried = 1
     fp32 = ctx.effective_precision() == "fp32"

@@ -433,7 +433,8 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
 // taking all pairs of a group together.
 static bool conv_use(const lelph_ctx* c, ConvGeo* g)
 {
-    if (c->conv_off || !conv_geo(c, g)) return false;
+    if (c->local_form == LELPH_FORM_BOX || c->conv_off || !conv_geo(c, g)) return false;
+    if (c->local_form == LELPH_FORM_SPHERE) return true;
     const lelph_lattice& L = c->lat;
     const int prec = effective_precision(c), nb = L.nbnds;
     // a pair whose box product takes less than some 100 us

@@ -205,6 +205,7 @@ struct lelph_ctx
     // the k+q box and the umklapp vector its consumer applies
     bool box_defer = false;
     bool conv_off = false; // a sphere that the sphere form does not take was met
+    int local_form = LELPH_FORM_AUTO;
     const void* kq_view = nullptr;
     int kq_g0[3] = {0, 0, 0};
 
@@ -1270,6 +1271,22 @@ int lelph_get_tuning(lelph_ctx* c, lelph_tuning* t)
 {
     if (!c || !t) return LELPH_ERR_ARG;
     *t = c->tune;
+    return LELPH_OK;
+}
+
+int lelph_set_local_form(lelph_ctx* c, int form)
+{
+    if (!c || form < LELPH_FORM_AUTO || form > LELPH_FORM_SPHERE) return LELPH_ERR_ARG;
+    c->local_form = form;
+    return LELPH_OK;
+}
+
+int lelph_get_local_form(lelph_ctx* c, int* requested, int* used)
+{
+    if (!c) return LELPH_ERR_ARG;
+    ConvGeo geo;
+    if (requested) *requested = c->local_form;
+    if (used) *used = conv_use(c, &geo) ? LELPH_FORM_SPHERE : LELPH_FORM_BOX;
     return LELPH_OK;
 }
 

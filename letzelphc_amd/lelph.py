@@ -19,8 +19,8 @@ import os
 
 import numpy as np
 
-from .abi import (KERNELS, PRECISIONS, Lattice, LongRange, LrParams, Pair, Pseudo, Symmetry,
-                  Tuning, c_double_p, c_int_p, dptr, i64ptr, pack_system)
+from .abi import (KERNELS, LOCAL_FORMS, PRECISIONS, Lattice, LongRange, LrParams, Pair, Pseudo,
+                  Symmetry, Tuning, c_double_p, c_int_p, dptr, i64ptr, pack_system)
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "liblelph_hip.so")
@@ -28,6 +28,7 @@ LIB_PATH = os.path.join(HERE, "liblelph_hip.so")
 EXPORTS = [
     "lelph_create", "lelph_destroy", "lelph_strerror", "lelph_set_precision",
     "lelph_get_precision", "lelph_elph_q_rotate_noalloc", "lelph_set_tuning", "lelph_get_tuning",
+    "lelph_set_local_form", "lelph_get_local_form",
     "lelph_multi_create", "lelph_multi_run", "lelph_multi_timings", "lelph_multi_destroy",
     "lelph_get_device_count", "lelph_upload_wfc", "lelph_create_vlocg_table",
     "lelph_dvlocq", "lelph_set_dvscf", "lelph_get_dvscf", "lelph_elph_local",
@@ -71,6 +72,8 @@ def lib():
         L.lelph_get_precision.argtypes = [C.c_void_p, c_int_p, c_int_p]
         L.lelph_set_tuning.argtypes = [C.c_void_p, C.POINTER(Tuning)]
         L.lelph_get_tuning.argtypes = [C.c_void_p, C.POINTER(Tuning)]
+        L.lelph_set_local_form.argtypes = [C.c_void_p, C.c_int]
+        L.lelph_get_local_form.argtypes = [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int)]
         L.lelph_multi_create.argtypes = [C.c_int, C.POINTER(C.c_void_p), c_double_p,
                                          C.POINTER(C.c_int64), C.POINTER(C.POINTER(Pair)),
                                          C.c_int, C.POINTER(C.c_void_p)]
@@ -219,6 +222,16 @@ class Context:
         _check(lib().lelph_get_tuning(self.h, C.byref(t)), "lelph_get_tuning")
         return {"split_target": t.split_target, "fft_lines": t.fft_lines,
                 "fp32_form": t.fp32_form, "ctile": t.ctile, "nl_form": t.nl_form}
+
+    def set_local_form(self, form: str):
+        """the form of the local part: "auto", "box" or "sphere" """
+        _check(lib().lelph_set_local_form(self.h, LOCAL_FORMS[form]), "lelph_set_local_form")
+
+    def local_form(self) -> str:
+        """the form that calls take as the context stands ("box" or "sphere")"""
+        used = C.c_int(0)
+        _check(lib().lelph_get_local_form(self.h, None, C.byref(used)), "lelph_get_local_form")
+        return {v: k for k, v in LOCAL_FORMS.items()}[used.value]
 
     def upload_wfc(self, ik, wfc, gvec, Fk=None):
         wfc = np.ascontiguousarray(wfc, np.complex128)

@@ -7,7 +7,8 @@ one-wave-per-tile split kernel.  The cases cover what its tiling pads: a
 mode count that is not a multiple of four (the last group of four modes
 has two padding modes whose results are not stored), band counts that are
 not multiples of 16 (rows) or 128 (columns, two column tiles at 136 bands),
-and two spins with a spin-resolved potential.
+and two spins with a spin-resolved potential.  The box form, which that kernel
+belongs to, is pinned; "auto" is what these small cells run by default.
 
 Bars: bf16x3 |dg|max/|g|max <= 1e-6 against the oracle; the FP64 path of the
 same context <= 1e-10.
@@ -34,7 +35,8 @@ CASES = {
 
 @pytest.mark.parametrize("case", list(CASES))
 @pytest.mark.parametrize("kminusq", [False, True])
-def test_headline_bf16x3(case, kminusq):
+@pytest.mark.parametrize("form", ["box", "auto"])
+def test_headline_bf16x3(case, kminusq, form):
     s = synth.tiny(**CASES[case])
     n = int(np.prod(s.fft_dims))
     # the producer/consumer kernel's conditions
@@ -45,10 +47,11 @@ def test_headline_bf16x3(case, kminusq):
     O.set_threads(8)
     dv = o.dv_total(0)
     ref = o.compute_elphq(0, dv, non_loc=True, kminusq=kminusq)
-    say(f"case: headline bf16x3 {case} kminusq={kminusq} nb={s.nbnds} nm={s.nmodes} "
+    say(f"case: headline bf16x3 {case} {form} kminusq={kminusq} nb={s.nbnds} nm={s.nmodes} "
         f"nspin={s.nspin} N={n}")
     ctx = lelph.Context(s, "fp64")
     try:
+        ctx.set_local_form(form)
         ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
         g64 = ctx.compute_elphq(s.qpts[0], non_loc=True, kminusq=kminusq)
         ctx.set_precision("bf16x3")

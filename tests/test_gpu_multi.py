@@ -15,6 +15,8 @@ precision over all tiles, the rest, captured in a HIP graph and replayed.
   FP32 cells 1e-6);
 - the autotuner's candidates reproduce the default g (bit for bit, or to
   rounding for the K-split count).
+In the form of the local part that the sizes choose (most cells: the sphere
+form) and with every cell in the box form (the work queues).
 """
 import os
 
@@ -29,12 +31,13 @@ from .util import rel_err, say
 pytestmark = [pytest.mark.gpu, pytest.mark.timeout(600)]
 
 
-@pytest.fixture(scope="module")
-def cells(tmp_path_factory):
+@pytest.fixture(scope="module", params=["auto", "box"])
+def cells(request, tmp_path_factory):
     cs = synth.config_c3()
     jobs = []
     for i, s in enumerate(cs):
         ctx = lelph.Context(s, "fp64" if i % 2 == 0 else "fp32")
+        ctx.set_local_form(request.param)
         ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
         jobs.append((ctx, s.qpts[0], synth.kq_pairs(s, 0)))
     cache = str(tmp_path_factory.mktemp("tune") / "tune.json")
@@ -56,7 +59,10 @@ def test_multi_bit_identical_to_cell_batches(cells):
     gm = [g.copy() for g in m.run()]
     _, gs = batch.run_sequential(jobs)
     _, gp = batch.run_pairwise(jobs)
-    say(f"  timings {m.timings()}")
+    t = m.timings()
+    say(f"  timings {t}")
+    if all(ctx.local_form() == "box" for ctx, _, _ in jobs):
+        assert t["items_fp64"] > 0 and t["items_fp32"] > 0
     for i, (a, b, c) in enumerate(zip(gm, gs, gp)):
         e = rel_err(a, c)
         say(f"  cell {i} {cs[i].fft_dims}: vs per-cell batch max |d| = "
@@ -99,11 +105,15 @@ def test_multi_vs_oracle(cells):
 
 def test_autotune_candidates_bit_identical(cells):
     """a forced re-tune of two cells (one per precision): tune() raises if
-    a candidate changes g beyond its bound; the cache records the choice"""
+    a candidate changes g beyond its bound; the cache records the choice.  A
+    cell in the sphere form, where the knobs change nothing, is timed once."""
     cs, jobs, _, cache = cells
     c = autotune.load_cache(cache)
     for i in (2, 3):
         ctx, q, pairs = jobs[i]
         r = autotune.tune(ctx, pairs, q, cache=c, force=True)
         say(f"  cell {i}: {r}")
-        assert autotune.shape_key(ctx) in c
+        if ctx.local_form() == "box":
+            assert r["tried"] > 1 and autotune.shape_key(ctx) in c
+        else:
+            assert r["tried"] == 1 and not any(r["tuning"].values())

@@ -3,7 +3,8 @@ potential (element-wise staging) and an FP32 collinear cell (separate
 staging) in the same work queue, an FP64 two-spin cell, a cell with no
 pairs, and a one-pair FP32 cell with its own contraction tile (a second
 FP32 queue).  Every cell's g is bit-identical to its own lelph_gkq_batch,
-replay after replay."""
+replay after replay.  In the box form, which fills the queues, and in the
+form that the sizes choose."""
 import numpy as np
 import pytest
 
@@ -22,7 +23,8 @@ CELLS = [
 ]
 
 
-def test_multi_mixed_cells():
+@pytest.mark.parametrize("form", ["box", "auto"])
+def test_multi_mixed_cells(form):
     jobs, ctxs = [], []
     try:
         for name, kw, prec, npair, ctile in CELLS:
@@ -30,6 +32,7 @@ def test_multi_mixed_cells():
             ctx = lelph.Context(s, prec)
             ctxs.append(ctx)
             ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
+            ctx.set_local_form(form)
             if ctile:
                 ctx.set_tuning(ctile=ctile)
             pairs = synth.kq_pairs(s, 0)
@@ -41,7 +44,9 @@ def test_multi_mixed_cells():
         m = lelph.MultiBatch(jobs)
         try:
             t = m.timings()
-            say(f"  items fp64 {t['items_fp64']}, fp32 {t['items_fp32']}")
+            say(f"  {form}: items fp64 {t['items_fp64']}, fp32 {t['items_fp32']}")
+            if form == "box":
+                assert t["items_fp64"] > 0 and t["items_fp32"] > 0
             refs = [ctx.gkq_batch(p, qpt=q) if len(p) else None for ctx, q, p in jobs]
             for rep in range(3):
                 out = m.run()

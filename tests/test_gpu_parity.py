@@ -36,6 +36,21 @@ def c0ctx(c0):
     ctx.close()
 
 
+@pytest.fixture(params=["auto", "box"])
+def form(request):
+    """the form of the local part: the one that the sizes choose (cells of
+    these sizes: the sphere form), and the box form"""
+    return request.param
+
+
+@pytest.fixture
+def c0form(c0ctx, form):
+    c0ctx.set_local_form(form)
+    assert c0ctx.local_form() == ("sphere" if form == "auto" else "box")
+    yield c0ctx
+    c0ctx.set_local_form("auto")
+
+
 def test_vloc_table(c0, c0ctx):
     s, o, _ = c0
     say("case: V_loc(G) table c0")
@@ -63,11 +78,11 @@ def test_dvscf_total(c0, c0ctx):
 
 
 @pytest.mark.parametrize("ip", [0, 1, 3, 17])
-def test_local_fp64(c0, c0ctx, ip):
+def test_local_fp64(c0, c0form, ip):
     s, o, dv = c0
     pr = synth.kq_pairs(s, 0)[ip]
     say(f"case: elph_local fp64 c0 pair {pr}")
-    g = c0ctx.elph_local(*pr)
+    g = c0form.elph_local(*pr)
     ref = o.elph_local(0, *pr, dv)
     assert rel_err(g, ref) < TOL64
 
@@ -83,35 +98,35 @@ def test_nonlocal_fp64(c0, c0ctx, ip):
     assert rel_err(g - base, ref - base) < TOL64
 
 
-def test_compute_elphq_fp64(c0, c0ctx):
+def test_compute_elphq_fp64(c0, c0form):
     s, o, dv = c0
     say("case: compute_elphq fp64 c0 all k")
-    g = c0ctx.compute_elphq(s.qpts[0], non_loc=True, kminusq=False)
+    g = c0form.compute_elphq(s.qpts[0], non_loc=True, kminusq=False)
     ref = o.compute_elphq(0, dv, non_loc=True, kminusq=False)
     assert rel_err(g, ref) < TOL64
 
 
-def test_compute_elphq_kminusq(c0, c0ctx):
+def test_compute_elphq_kminusq(c0, c0form):
     s, o, dv = c0
     say("case: compute_elphq fp64 c0 yambo convention")
-    g = c0ctx.compute_elphq(s.qpts[0], non_loc=True, kminusq=True)
+    g = c0form.compute_elphq(s.qpts[0], non_loc=True, kminusq=True)
     ref = o.compute_elphq(0, dv, non_loc=True, kminusq=True, k_first=0, k_count=16)
     assert rel_err(g[:16], ref) < TOL64
 
 
 @pytest.mark.parametrize("prec", ["fp32", "bf16x6", "bf16x3"])
-def test_compute_elphq_reduced(c0, c0ctx, prec):
+def test_compute_elphq_reduced(c0, c0form, prec):
     """FP32 and split-product forms at 1e-6.  c0's 8 bands are off the
     producer/consumer path, so a bf16x3 request runs as bf16x6 there."""
     s, o, dv = c0
     say(f"case: compute_elphq {prec} c0 all k")
-    c0ctx.set_precision(prec)
+    c0form.set_precision(prec)
     try:
-        eff = c0ctx.effective_precision()
+        eff = c0form.effective_precision()
         assert eff == ("bf16x6" if prec == "bf16x3" else prec)
-        g = c0ctx.compute_elphq(s.qpts[0], non_loc=True)
+        g = c0form.compute_elphq(s.qpts[0], non_loc=True)
     finally:
-        c0ctx.set_precision("fp64")
+        c0form.set_precision("fp64")
     ref = o.compute_elphq(0, dv, non_loc=True)
     err = rel_err(g, ref)
     say(f"  {prec} (runs as {eff}): |dg|/|g|max = {err:.3e}")
@@ -120,7 +135,7 @@ def test_compute_elphq_reduced(c0, c0ctx, prec):
 
 @pytest.mark.parametrize("prec", ["fp32", "bf16x6", "bf16x3"])
 @pytest.mark.parametrize("kind", ["spin2", "spinor_nmag1", "spinor_nmag4", "soc_nmag4"])
-def test_tiny_variants_reduced(kind, prec):
+def test_tiny_variants_reduced(kind, prec, form):
     """FP32 and split-product contractions on the spin / spinor / 2x2
     potential branches (the split kernel's element-wise staging path for
     spinors and nmag 4, spin-resolved dV for nmag 2), against the oracle."""
@@ -135,9 +150,10 @@ def test_tiny_variants_reduced(kind, prec):
         kw.update(nspinor=2, nmag=4, soc=True, syms="cubic", q=(0.0, 0.5, 0.0))
     s = synth.tiny(**kw)
     o = O.OracleSystem(s)
-    say(f"case: tiny {kind} {prec}")
+    say(f"case: tiny {kind} {prec} {form}")
     ctx = lelph.Context(s, "fp64")
     try:
+        ctx.set_local_form(form)
         ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
         ctx.set_precision(prec)
         g = ctx.compute_elphq(s.qpts[0], non_loc=True)
@@ -151,7 +167,7 @@ def test_tiny_variants_reduced(kind, prec):
 
 @pytest.mark.parametrize("kind", ["spin2", "spinor_nmag1", "spinor_nmag4", "cubic_syms",
                                   "bare", "dfpt_local", "slab_2d", "soc", "soc_nmag4"])
-def test_tiny_variants(kind):
+def test_tiny_variants(kind, form):
     kw = dict(nbnds=4)
     kernel = "dfpt"
     if kind == "spin2":
@@ -172,8 +188,9 @@ def test_tiny_variants(kind):
         kw.update(nspinor=2, nmag=4, soc=True, syms="cubic", q=(0.0, 0.5, 0.0))
     s = synth.tiny(**kw)
     o = O.OracleSystem(s)
-    say(f"case: tiny {kind}")
+    say(f"case: tiny {kind} {form}")
     ctx = lelph.Context(s, "fp64")
+    ctx.set_local_form(form)
     ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel=kernel)
     dv = o.dv_total(0, kernel=kernel)
     assert rel_err(ctx.get_dvscf(), dv) < TOL64
@@ -222,7 +239,7 @@ def test_error_paths():
     ctx.close()
 
 
-def test_c1_symmetry_pairs():
+def test_c1_symmetry_pairs(form):
     """The layered c1 cell (45x45x216, 12 operations incl. time reversal),
     16 bands: pairs whose k and k+q need non-trivial and time-reversed
     operations, FP64 to 1e-10 and the reduced variants (generic, unaligned
@@ -237,9 +254,10 @@ def test_c1_symmetry_pairs():
         if key not in seen:
             seen.add(key)
             pick.append(pr)
-    say(f"case: c1 pairs {pick}")
+    say(f"case: c1 pairs {pick} {form}")
     dv = o.dv_total(0)
     ctx = lelph.Context(s, "fp64")
+    ctx.set_local_form(form)
     ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
     try:
         for pr in pick:
@@ -359,7 +377,7 @@ def test_chain_sides_counts():
 
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32", "bf16x3", "bf16x6"])
-def test_batch_gamma_self_loops(prec):
+def test_batch_gamma_self_loops(prec, form):
     """At q = 0 every pair's k+q side is its own k side (a cycle of one
     pair): a batch transforms one psi side per pair, takes the k+q box over
     from the pair's own psi_k box (a copy in FP64 / FP32, read as it is by
@@ -369,9 +387,10 @@ def test_batch_gamma_self_loops(prec):
     o = O.OracleSystem(s)
     pairs = synth.kq_pairs(s, 0)
     assert all(ikq == ik and kqs == ks for (ikq, ik, kqs, ks) in pairs)
-    say(f"case: q = 0 batch {prec}, {len(pairs)} self-loop pairs")
+    say(f"case: q = 0 batch {prec} {form}, {len(pairs)} self-loop pairs")
     ctx = lelph.Context(s, "fp64")
     try:
+        ctx.set_local_form(form)
         ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
         ctx.set_precision(prec)
         gb = ctx.gkq_batch(pairs, non_loc=True, qpt=s.qpts[0])
@@ -389,7 +408,7 @@ def test_batch_gamma_self_loops(prec):
 
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("bf16x3", 0.0)])
-def test_batch_shuffled_with_repeats(c0, c0ctx, prec, tol):
+def test_batch_shuffled_with_repeats(c0, c0form, prec, tol):
     """A batch in random order with repeated pairs: repeats compete for the
     same chain links, so heads, cycle closes and mirrored non-local sides
     fall in irregular places; every pair's g equals its pair-by-pair g (bit
@@ -402,13 +421,13 @@ def test_batch_shuffled_with_repeats(c0, c0ctx, prec, tol):
     pairs = [pairs[i] for i in rng.permutation(len(pairs))]
     want_sides = _chain_sides(pairs)
     say(f"case: shuffled batch with repeats {prec}, {len(pairs)} pairs, sides {want_sides}")
-    c0ctx.set_precision(prec)
+    c0form.set_precision(prec)
     try:
-        gb = c0ctx.gkq_batch(pairs, non_loc=True, qpt=s.qpts[0])
-        sides = c0ctx.last_timings()["box_sides"]
-        one = {p: c0ctx.gkq(*p, non_loc=True, qpt=s.qpts[0]) for p in set(pairs)}
+        gb = c0form.gkq_batch(pairs, non_loc=True, qpt=s.qpts[0])
+        sides = c0form.last_timings()["box_sides"]
+        one = {p: c0form.gkq(*p, non_loc=True, qpt=s.qpts[0]) for p in set(pairs)}
     finally:
-        c0ctx.set_precision("fp64")
+        c0form.set_precision("fp64")
     assert sides == want_sides
     ref = np.stack([one[p] for p in pairs])
     if tol == 0.0:
@@ -419,7 +438,7 @@ def test_batch_shuffled_with_repeats(c0, c0ctx, prec, tol):
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", TOL32), ("bf16x3", TOL32)])
 @pytest.mark.parametrize("kminusq", [False, True])
-def test_batch_box_reuse(c0, c0ctx, prec, tol, kminusq):
+def test_batch_box_reuse(c0, c0form, prec, tol, kminusq):
     """A batch walks k -> k+q chains and takes each pair's k box from the
     previous pair's k+q box, shifted back by its umklapp vector, and the
     last pair of a closed cycle its k+q box from the head's k box, shifted
@@ -434,14 +453,14 @@ def test_batch_box_reuse(c0, c0ctx, prec, tol, kminusq):
     say(f"case: box reuse {prec} kminusq={kminusq} pairs={len(pairs)} links={links} "
         f"sides={want_sides}")
     assert links >= len(pairs) // 2
-    c0ctx.set_precision(prec)
+    c0form.set_precision(prec)
     try:
-        gb = c0ctx.gkq_batch(pairs, non_loc=True, qpt=s.qpts[0])
-        sides = c0ctx.last_timings()["box_sides"]
-        one = np.stack([c0ctx.gkq(*p, non_loc=True, qpt=s.qpts[0]) for p in pairs])
-        assert c0ctx.last_timings()["box_sides"] == 2
+        gb = c0form.gkq_batch(pairs, non_loc=True, qpt=s.qpts[0])
+        sides = c0form.last_timings()["box_sides"]
+        one = np.stack([c0form.gkq(*p, non_loc=True, qpt=s.qpts[0]) for p in pairs])
+        assert c0form.last_timings()["box_sides"] == 2
     finally:
-        c0ctx.set_precision("fp64")
+        c0form.set_precision("fp64")
     assert sides == want_sides
     err = rel_err(gb, one)
     say(f"  batch vs pair by pair: {err:.3e}")

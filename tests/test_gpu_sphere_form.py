@@ -46,6 +46,7 @@ def test_grids(fft):
         ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
         for prec in ("fp64", "fp32"):
             ctx.set_precision(prec)
+            assert ctx.local_form() == ("box" if {13, 22, 26} & set(fft) else "sphere")
             errs[prec] = rel_err(ctx.gkq_batch(pick, qpt=s.qpts[0]), ref)
     finally:
         ctx.close()
@@ -78,6 +79,7 @@ def test_bands_and_spin(case, nb, fft):
         ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
         for prec in ("fp64", "fp32"):
             ctx.set_precision(prec)
+            assert ctx.local_form() == "sphere"
             one = np.stack([ctx.elph_local(*p) for p in pairs[:2]])
             bat = ctx.gkq_batch(pairs, non_loc=False, qpt=s.qpts[0])[:2]
             # a pair's sums do not depend on what it is batched with

@@ -5,7 +5,8 @@ the same operands in the same order for each g element and keeps the K
 splits of the wide tile, so g is bit-identical across shapes; each against
 the FP64 oracle (FP64 <= 1e-10, FP32 <= 1e-6).  Band counts that pad the
 tiles differently (8, 24, 40, 80), a spinor cell with the 2x2 potential
-(element-wise FP32 form) and a two-spin cell."""
+(element-wise FP32 form) and a two-spin cell.  The contraction belongs to the
+box form, which is pinned."""
 import numpy as np
 import pytest
 
@@ -36,6 +37,7 @@ def test_tile_shapes(case, prec):
     ref = [o.elph_local(0, *p, dv) for p in pairs]
     ctx = lelph.Context(s, prec)
     try:
+        ctx.set_local_form("box")
         ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
         gs = {}
         for ct in (0, 1, 2, 3, 4):

@@ -14,6 +14,9 @@ on the host cores in the same process.
   rotations and time-reversed operations, in both the k+q and k-q
   conventions, one pair by one and as a chained batch.
 
+Every precision in the form of the local part that its sizes choose, and in
+the box form where that is another one.
+
 Bars: FP64 |dg|max/|g|max <= 1e-10, FP32 / bf16x6 / bf16x3 <= 1e-6.
 """
 import os
@@ -32,6 +35,12 @@ pytestmark = [pytest.mark.gpu, pytest.mark.timeout(900)]
 TOL64 = 1e-10
 TOL32 = 1e-6
 PRECS = ("fp64", "fp32", "bf16x6", "bf16x3")
+
+
+def _forms(ctx):
+    """the forms to compare: the chosen one, and the box form"""
+    ctx.set_local_form("auto")
+    return ["auto"] if ctx.local_form() == "box" else ["auto", "box"]
 
 
 def _cores():
@@ -63,9 +72,11 @@ def c2():
         dv_err = rel_err(ctx.get_dvscf(), dv)
         for prec in PRECS:
             ctx.set_precision(prec)
-            res[prec] = (ctx.effective_precision(),
-                         ctx.gkq_batch(chain, non_loc=True, qpt=s.qpts[0]))
-            say(f"  c2 batch {prec} done")
+            for form in _forms(ctx):
+                ctx.set_local_form(form)
+                res[prec, form] = (ctx.effective_precision(),
+                                   ctx.gkq_batch(chain, non_loc=True, qpt=s.qpts[0]))
+                say(f"  c2 batch {prec} {form} ({ctx.local_form()}) done")
     finally:
         ctx.close()
     yield s, chain, futs, res, dv_err
@@ -84,23 +95,22 @@ def test_c2_chain_vs_oracle(c2, i):
     s, chain, futs, res, _ = c2
     say(f"case: c2 pair {chain[i]} ({'umklapp k+q' if i == 1 else 'shifted box reuse'})")
     ref = futs[i].result()
-    for prec in PRECS:
-        eff, g = res[prec]
+    for (prec, form), (eff, g) in res.items():
         err = rel_err(g[i], ref)
-        say(f"  c2 {prec} (runs as {eff}): |dg|/|g|max = {err:.3e}")
+        say(f"  c2 {prec} {form} (runs as {eff}): |dg|/|g|max = {err:.3e}")
         assert eff == prec
-        assert err < (TOL64 if prec == "fp64" else TOL32), prec
+        assert err < (TOL64 if prec == "fp64" else TOL32), (prec, form)
 
 
 def test_c2_first_pair_consistent(c2):
     """The first pair of the batch (both boxes transformed) against the
     FP64 result of the same batch: the reduced forms stay at 1e-6."""
     _, _, _, res, _ = c2
-    g64 = res["fp64"][1]
-    for prec in PRECS[1:]:
-        err = rel_err(res[prec][1][0], g64[0])
-        say(f"  c2 first pair {prec} vs FP64: {err:.3e}")
-        assert err < TOL32
+    g64 = res["fp64", "auto"][1]
+    for (prec, form), (_, g) in res.items():
+        err = rel_err(g[0], g64[0])
+        say(f"  c2 first pair {prec} {form} vs FP64: {err:.3e}")
+        assert err < (TOL64 if prec == "fp64" else TOL32)
 
 
 def _c1_pick(s, iq, kminusq):
@@ -145,11 +155,13 @@ def test_c1_full(c1, iq, kminusq):
         for prec in PRECS:
             ctx.set_precision(prec)
             eff = ctx.effective_precision()
-            for pr, ref in zip(pick, refs):
-                g = ctx.gkq(*pr, qpt=s.qpts[iq])
-                err = rel_err(g, ref)
-                say(f"  {pr} {prec} (runs as {eff}): {err:.3e}")
-                assert err < (TOL64 if prec == "fp64" else TOL32), (pr, prec)
+            for form in _forms(ctx):
+                ctx.set_local_form(form)
+                for pr, ref in zip(pick, refs):
+                    g = ctx.gkq(*pr, qpt=s.qpts[iq])
+                    err = rel_err(g, ref)
+                    say(f"  {pr} {prec} {form} (runs as {eff}): {err:.3e}")
+                    assert err < (TOL64 if prec == "fp64" else TOL32), (pr, prec, form)
     finally:
         ctx.close()
 
@@ -167,9 +179,11 @@ def test_c1_batch_chain(c1):
         ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
         for prec in ("fp64", "bf16x3"):
             ctx.set_precision(prec)
-            g = ctx.gkq_batch(synth.kq_pairs(s, 0), non_loc=True, qpt=s.qpts[0])
-            err = rel_err(g[:12], ref)
-            say(f"  c1 batch {prec}: {err:.3e}")
-            assert err < (TOL64 if prec == "fp64" else TOL32)
+            for form in _forms(ctx):
+                ctx.set_local_form(form)
+                g = ctx.gkq_batch(synth.kq_pairs(s, 0), non_loc=True, qpt=s.qpts[0])
+                err = rel_err(g[:12], ref)
+                say(f"  c1 batch {prec} {form}: {err:.3e}")
+                assert err < (TOL64 if prec == "fp64" else TOL32)
     finally:
         ctx.close()
