@@ -595,20 +595,25 @@ int lelph_interp_timings(lelph_ctx* ctx, double* ms, int n);
 
 /* Device time of the last elph_local / nonlocal / gkq / batch call, summed
  * over its pairs (HIP events), milliseconds:
- *   [0] sphere scatter + backward FFTs of psi_k and psi_k+q
- *   [1] local contraction kernel (the MFMA GEMM)
+ *   [0] sphere scatter + backward FFTs of psi_k and psi_k+q (sphere form:
+ *       both spheres, the psi_k boxes)
+ *   [1] local contraction kernel (the MFMA GEMM; sphere form: the transforms
+ *       of dV psi and the product over the sphere)
  *   [2] split-K reduction and 1/N
  *   [3] non-local part; in a batch, where it runs on a second stream beside
  *       the local parts, the time from the end of the pair's local part to
  *       the end of its non-local part
  *   [4] total device time per pair (start of its local part to the end of
- *       both parts; overlapping pairs of a batch count their overlap twice)
+ *       both parts; overlapping pairs of a batch count their overlap twice;
+ *       sphere form: per group of pairs)
  *   [5] number of (k,k+q) pairs
- *   [6] number of psi sides transformed (sphere scatter + backward FFT); a
- *       batch takes the others over along k -> k+q chains with the shift
- *       theorem: a pair's psi_k box is the psi_k+q box of the pair before
- *       it, and the last pair of a closed cycle (k + nq = k + G) takes its
- *       psi_k+q box from the first pair's psi_k box
+ *   [6] number of psi boxes formed (sphere scatter + backward FFT).  Box
+ *       form: of both sides; a batch takes the others over along k -> k+q
+ *       chains with the shift theorem: a pair's psi_k box is the psi_k+q box
+ *       of the pair before it, and the last pair of a closed cycle
+ *       (k + nq = k + G) takes its psi_k+q box from the first pair's psi_k
+ *       box.  Sphere form: of the k sides only, each distinct one once per
+ *       group of pairs that go through the steps together
  * n: number of entries wanted (<= 8). */
 int lelph_last_timings(lelph_ctx* ctx, double* ms, int n);
 

@@ -364,6 +364,7 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
                  geo.r1[1], geo.r2[1], geo.r2[2]};
     LELPH_TRY(conv_box_plane_launch<T>(geo.box, nx8 * geo.nrows * nk, st, ds + np, ba, pb, Wy,
                                        Wz));
+    c->box_sides += nk;
     if (ev) HIP_TRY(hipEventRecord(ev[1], st));
     // dV psi to the sphere, a chunk of modes at a time
     PlaneArgs pc{geo.conv.lds.rows, geo.conv.lds.prow, geo.conv.lds.tw,

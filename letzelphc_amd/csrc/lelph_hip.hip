@@ -972,7 +972,6 @@ static int run_local_any(lelph_ctx* c, const double* qpt, const lelph_pair& pr, 
     if (conv_use(c, &geo))
     {
         LELPH_TRY(conv_prepare(c, geo));
-        c->box_sides = 2;
         return conv_group_local(c, geo, conv_group(c, geo, 1), c->cv, c->cv.desc, true, qpt, &pr,
                                 1, g, c->stream, ev);
     }
@@ -1765,29 +1764,6 @@ int lelph_gkq(lelph_ctx* c, const double qpt[3], int ikq, int ik, int kqsym, int
 }
 
 extern "C++" {
-// psi sides that a walk along k -> k+q chains leaves: a head's two, one per
-// linked pair, none for the k+q side that closes a cycle on its head
-static int64_t chain_sides(const lelph_pair* pairs, const std::vector<int64_t>& order)
-{
-    int64_t n = 0;
-    const lelph_pair* head = nullptr;
-    const lelph_pair* prev = nullptr;
-    for (int64_t i : order)
-    {
-        const lelph_pair& p = pairs[i];
-        const bool link = prev && prev->ikq == p.ik && prev->kqsym == p.ksym;
-        if (!link)
-        {
-            head = &p;
-            ++n;
-        }
-        const bool close = head->ik == p.ikq && head->ksym == p.kqsym;
-        if (!close) ++n;
-        prev = &p;
-    }
-    return n;
-}
-
 // lelph_gkq_batch in the sphere form: groups of pairs, their non-local parts
 // on the second stream along the chains, each group's g copied out while
 // later groups compute
@@ -1814,7 +1790,7 @@ static int conv_batch(lelph_ctx* c, const ConvGeo& geo, const double* qpt, int64
                         ring + slot * slice * np + (p - p0) * slice, slice);
         return LELPH_OK;
     };
-    c->box_sides = chain_sides(pairs, order);
+    c->box_sides = 0;
     if (non_loc) nl_plan(c, pairs, order, np);
     std::vector<lelph_pair> grp((size_t)np);
     int64_t landed = 0;

@@ -365,6 +365,12 @@ def _chain_sides(pairs):
     return sides
 
 
+def _want_sides(form, pairs):
+    """psi boxes a batch forms: what the chains leave in the box form, every
+    distinct k side in the sphere form (these cells: one group of pairs)"""
+    return _chain_sides(pairs) if form == "box" else len({(p[1], p[3]) for p in pairs})
+
+
 def test_chain_sides_counts():
     """A chain a -> b -> c -> a (a closed cycle) needs three transforms, an
     open chain a -> b -> c four, a self-loop one, two disjoint pairs four."""
@@ -398,7 +404,7 @@ def test_batch_gamma_self_loops(prec, form):
         one = np.stack([ctx.gkq(*p, non_loc=True, qpt=s.qpts[0]) for p in pairs])
     finally:
         ctx.close()
-    assert sides == len(pairs)
+    assert sides == len(pairs)  # in either form
     assert np.array_equal(gb, one)
     dv = o.dv_total(0)
     ref = np.stack([o.add_nonlocal(0, *p, o.elph_local(0, *p, dv)) for p in pairs[:3]])
@@ -408,19 +414,20 @@ def test_batch_gamma_self_loops(prec, form):
 
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("bf16x3", 0.0)])
-def test_batch_shuffled_with_repeats(c0, c0form, prec, tol):
+def test_batch_shuffled_with_repeats(c0, c0form, form, prec, tol):
     """A batch in random order with repeated pairs: repeats compete for the
     same chain links, so heads, cycle closes and mirrored non-local sides
     fall in irregular places; every pair's g equals its pair-by-pair g (bit
     for bit in the split precisions, which build every box in k-side form)
-    and the batch transforms exactly the sides its chain walk leaves."""
+    and the batch transforms exactly the sides its chain walk leaves (sphere
+    form: every distinct k side)."""
     s, o, dv = c0
     rng = np.random.default_rng(5)
     base = synth.kq_pairs(s, 0)
     pairs = base + [base[i] for i in rng.choice(len(base), 12, replace=False)]
     pairs = [pairs[i] for i in rng.permutation(len(pairs))]
-    want_sides = _chain_sides(pairs)
-    say(f"case: shuffled batch with repeats {prec}, {len(pairs)} pairs, sides {want_sides}")
+    want_sides = _want_sides(form, pairs)
+    say(f"case: shuffled batch with repeats {prec} {form}, {len(pairs)} pairs, sides {want_sides}")
     c0form.set_precision(prec)
     try:
         gb = c0form.gkq_batch(pairs, non_loc=True, qpt=s.qpts[0])
@@ -438,19 +445,19 @@ def test_batch_shuffled_with_repeats(c0, c0form, prec, tol):
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", TOL32), ("bf16x3", TOL32)])
 @pytest.mark.parametrize("kminusq", [False, True])
-def test_batch_box_reuse(c0, c0form, prec, tol, kminusq):
+def test_batch_box_reuse(c0, c0form, form, prec, tol, kminusq):
     """A batch walks k -> k+q chains and takes each pair's k box from the
     previous pair's k+q box, shifted back by its umklapp vector, and the
     last pair of a closed cycle its k+q box from the head's k box, shifted
     by its own; pair by pair (every box transformed) gives the same g (the
     bf16 split precisions bit for bit).  The pairs go in reversed order so
     the batch has to rebuild the chains itself; it transforms exactly the
-    sides the chains leave."""
+    sides the chains leave (sphere form: every distinct k side)."""
     s, o, dv = c0
     pairs = synth.kq_pairs(s, 0, kminusq=kminusq)[::-1]
     links = _chain_links(pairs)
-    want_sides = _chain_sides(pairs)
-    say(f"case: box reuse {prec} kminusq={kminusq} pairs={len(pairs)} links={links} "
+    want_sides = _want_sides(form, pairs)
+    say(f"case: box reuse {prec} {form} kminusq={kminusq} pairs={len(pairs)} links={links} "
         f"sides={want_sides}")
     assert links >= len(pairs) // 2
     c0form.set_precision(prec)
@@ -458,7 +465,7 @@ def test_batch_box_reuse(c0, c0form, prec, tol, kminusq):
         gb = c0form.gkq_batch(pairs, non_loc=True, qpt=s.qpts[0])
         sides = c0form.last_timings()["box_sides"]
         one = np.stack([c0form.gkq(*p, non_loc=True, qpt=s.qpts[0]) for p in pairs])
-        assert c0form.last_timings()["box_sides"] == 2
+        assert c0form.last_timings()["box_sides"] == (2 if form == "box" else 1)
     finally:
         c0form.set_precision("fp64")
     assert sides == want_sides
