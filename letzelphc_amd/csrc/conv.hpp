@@ -723,14 +723,13 @@ struct ConvPair
     const void* dv;   // (nm, nmag, N)
     int side;         // k+q side
     void* line;       // (modes, sets of a launch, Nx, sticks) after the y step
-    void* c;          // (nm, sets, ld) on the sphere
-    z64* out;         // partials or g
+    void* c;          // (modes of a block, sets, ld) on the sphere
 };
 
 struct ConvArgs
 {
     int Nx, Ny, Nz, words;
-    int nm, v0, nv;   // modes in all, first and number of this launch
+    int vc, v0, nv;   // first mode that c holds, first and number of this launch
     int s0, ns;       // first set (spin, band, spinor) and number of this launch
     int nspin, nb, nspinor, nmag;
     int nzk_max, nst_max;
@@ -800,7 +799,7 @@ __device__ inline void conv_x_body(const ConvPair& pr, const SphSide& sd, const 
     {
         const auto in = gptr<T>::of(pr.line) + (row * N * nst + s0);
         const auto c = gptr<T>::of(pr.c) +
-                       ((a.v0 + row / a.ns) * nsets + a.s0 + row % a.ns) * sd.ld;
+                       ((a.v0 - a.vc + row / a.ns) * nsets + a.s0 + row % a.ns) * sd.ld;
         for (int t = tid; t < TS * R2; t += NT)
         {
             const int s = t % TS, j = t / TS;

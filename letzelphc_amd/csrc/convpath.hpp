@@ -34,6 +34,10 @@ static const int64_t CONV_LINE_BYTES = 1024ll << 20;
 // drift apart and miss, 3 %; 4: 2 % in starting blocks)
 static const int CONV_MODES = 8, CONV_SETS = 8;
 static const int64_t CONV_GROUP_BYTES = 2ll << 30;
+// bytes of a pair's coefficients on the k+q sphere, all sets of a block of
+// modes (144^3, 96 atoms, 480 bands would take 336 GB at once).  Beyond the
+// 96^3 cell's 3.6 GB: a block reads the psi boxes again.
+static const int64_t CONV_C_BYTES = 4ll << 30;
 static const int CONV_GROUP_PAIRS = 256;
 
 // threads of the blocks over planes: as many waves as leave the fewest idle
@@ -133,11 +137,11 @@ static bool conv_geo(const lelph_ctx* c, ConvGeo* g)
     return true;
 }
 
-// pairs that go through the steps together, and the modes and sets of a
-// plane launch
+// pairs that go through the steps together, the modes and sets of a plane
+// launch, and the modes of a block: transformed to the sphere, then contracted
 struct ConvGroup
 {
-    int np, nv, ns;
+    int np, nv, ns, nm;
 };
 
 static ConvGroup conv_group(const lelph_ctx* c, const ConvGeo& g, int64_t npairs)
@@ -156,18 +160,26 @@ static ConvGroup conv_group(const lelph_ctx* c, const ConvGeo& g, int64_t npairs
     p = std::min<int64_t>(p, 65535 / std::max(1, L.nspin) / 2);
     ConvGroup r;
     r.np = (int)std::max<int64_t>(1, p);
+    int64_t nm = L.nmodes; // several pairs: all modes are within a group's bytes
+    if (r.np == 1)
+    {
+        nm = std::max<int64_t>(1, CONV_C_BYTES / (item * g.nrows * g.ld));
+        if (nm > CONV_MODES) nm -= nm % CONV_MODES;
+        nm = std::min<int64_t>(nm, L.nmodes);
+    }
     // one pair: up to 8 modes share a psi plane, the sets fill the rest
-    int64_t nv = L.nmodes, ns = g.nrows;
+    int64_t nv = nm, ns = g.nrows;
     if (nv * ns * r.np > room)
     {
-        nv = std::min<int64_t>(L.nmodes, CONV_MODES);
+        nv = std::min<int64_t>(nm, CONV_MODES);
         nv = std::max<int64_t>(1, std::min(nv, room));
         ns = std::max<int64_t>(1, std::min<int64_t>(g.nrows, room / nv));
-        if (ns == g.nrows) nv = std::max<int64_t>(1, std::min<int64_t>(L.nmodes, room / ns));
+        if (ns == g.nrows) nv = std::max<int64_t>(1, std::min<int64_t>(nm, room / ns));
     }
     nv = std::max<int64_t>(1, std::min<int64_t>(nv, 500000 / ns)); // grid rows
     r.nv = (int)nv;
     r.ns = (int)ns;
+    r.nm = (int)nm;
     return r;
 }
 
@@ -212,15 +224,16 @@ struct ConvLayout
         s_line = row * Nx * g.nst;
         s_box = row * (size_t)ctx->nf;
         s_cl = item * (size_t)gr.ns * gr.nv * Nx * g.nst;
-        s_c = s_coef * L.nmodes;
+        s_c = s_coef * gr.nm;
         map = o_ph + per * ns;
         coef = s_coef * ns;
         line = std::max(s_line * (ns - np), s_cl * np);
         box = s_box * (ns - np);
         c = s_c * np;
-        const size_t gsz = (size_t)L.nmodes * L.nspin * L.nbnds * L.nbnds;
+        const size_t gsz = (size_t)gr.nm * L.nspin * L.nbnds * L.nbnds; // of a block
         part = g.nsplit > 1 ? sizeof(z64) * (size_t)g.nsplit * np * gsz : 0;
     }
+    size_t bytes() const { return map + coef + line + box + c + part; }
     int ensure(ConvBufs& b, hipStream_t st) const
     {
         LELPH_TRY(buf_grow(b.map, map, b.fixed, st));
@@ -301,14 +314,13 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
     const int ns = (int)sides.size(), nk = ns - np;
     const ConvLayout lay(c, geo, gr, np, ns);
     LELPH_TRY(lay.ensure(b, st));
-    const int64_t gsz = (int64_t)L.nmodes * L.nspin * L.nbnds * L.nbnds;
-    char* m0 = b.map.as<char>();
+    char* mp = b.map.as<char>();
     for (int i = 0; i < ns; ++i)
     {
         SphSide& s = sides[i];
         s.ld = (int)(cdiv(s.npw, 16) * 16);
-        s.mask = reinterpret_cast<unsigned*>(m0 + lay.n_mask * i);
-        char* m = m0 + lay.o_ph + lay.per * i;
+        s.mask = reinterpret_cast<unsigned*>(mp + lay.n_mask * i);
+        char* m = mp + lay.o_ph + lay.per * i;
         s.cnt = reinterpret_cast<int*>(m + lay.per - 256);
         s.ph = reinterpret_cast<z64*>(m);
         s.idx = reinterpret_cast<int*>(m += lay.s_ph);
@@ -342,7 +354,7 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
     const z64 *Wx = axis_tw<double>(c->ax[0]), *Wy = axis_tw<double>(c->ax[1]),
               *Wz = axis_tw<double>(c->ax[2]);
 
-    LELPH_TRY(zero_async(m0, lay.n_mask * ns, st));
+    LELPH_TRY(zero_async(mp, lay.n_mask * ns, st));
     LELPH_TRY(conv_maps_launch(ns, geo.npw, st, ds, Nx, Ny, Nz, geo.words, geo.nzk, geo.nst,
                                c->d_err));
     const int64_t nsets = (int64_t)L.nspin * L.nbnds;
@@ -369,48 +381,54 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
     // dV psi to the sphere, a chunk of modes at a time
     PlaneArgs pc{geo.conv.lds.rows, geo.conv.lds.prow, geo.conv.lds.tw,
                  geo.r1[1], geo.r2[1], geo.r2[2]};
-    for (int64_t vs = 0; vs < cdiv(L.nmodes, nv) * cdiv(geo.nrows, nset); ++vs)
+    const int64_t es = (int64_t)L.nspin * L.nbnds * L.nbnds;
+    for (int m0 = 0; m0 < L.nmodes; m0 += gr.nm)
     {
-        // sets outside, modes inside: the psi boxes of the sets stay cached
-        const int v0 = (int)(vs % cdiv(L.nmodes, nv)) * nv;
-        ConvArgs a{};
-        a.Nx = Nx;
-        a.Ny = Ny;
-        a.Nz = Nz;
-        a.words = geo.words;
-        a.nm = L.nmodes;
-        a.v0 = v0;
-        a.nv = std::min(nv, L.nmodes - v0);
-        a.s0 = (int)(vs / cdiv(L.nmodes, nv)) * nset;
-        a.ns = (int)std::min<int64_t>(nset, geo.nrows - a.s0);
-        a.nspin = L.nspin;
-        a.nb = L.nbnds;
-        a.nspinor = L.nspinor;
-        a.nmag = nmag_eff;
-        a.nzk_max = geo.nzk;
-        a.nst_max = geo.nst;
-        const int64_t planes = (int64_t)a.ns * Nx * a.nv * np;
-        a.sper = (int)std::max<int64_t>(1, std::min<int64_t>(CONV_SETS, planes / 1024));
-        const int64_t blocks = nx8 * a.nv * cdiv(a.ns, a.sper) * np;
-        if (geo.square)
-            LELPH_TRY(conv_square_launch<T>(geo.sqlds, blocks, st, dp, ds, a, Wz));
-        else
-            LELPH_TRY(conv_plane_launch<T>(geo.two, geo.conv, blocks, st, dp, ds, a, pc, Wy, Wz));
-        const int64_t rows = (int64_t)a.ns * a.nv;
-        a.rows_per_block =
-            (int)std::max<int64_t>(1, std::min<int64_t>(8, rows * tiles * np / 4096));
-        LELPH_TRY(conv_x_launch<T>(geo.xcls, geo.xlds,
-                                   dim3(tiles, (unsigned)cdiv(rows, a.rows_per_block),
-                                        (unsigned)np),
-                                   st, dp, ds, a, Wx));
-    }
-    LELPH_TRY(sph_gemm_launch<T>(geo.nsplit, np, st, dp, ds, L.nmodes, L.nspin, L.nbnds,
-                                 L.nspinor, 1.0 / (double)c->nf,
-                                 geo.nsplit > 1 ? b.part.as<z64>() : g));
-    if (ev) HIP_TRY(hipEventRecord(ev[2], st));
-    if (geo.nsplit > 1)
-    {
-        LELPH_TRY(reduce_parts(b.part.as<z64>(), geo.nsplit, gsz * np, 1.0 / (double)c->nf, g, st));
+        const int nm = std::min(gr.nm, L.nmodes - m0);
+        const int64_t nvs = cdiv(nm, nv);
+        for (int64_t vs = 0; vs < nvs * cdiv(geo.nrows, nset); ++vs)
+        {
+            // sets outside, modes inside: the psi boxes of the sets stay cached
+            ConvArgs a{};
+            a.Nx = Nx;
+            a.Ny = Ny;
+            a.Nz = Nz;
+            a.words = geo.words;
+            a.vc = m0;
+            a.v0 = m0 + (int)(vs % nvs) * nv;
+            a.nv = std::min(nv, m0 + nm - a.v0);
+            a.s0 = (int)(vs / nvs) * nset;
+            a.ns = (int)std::min<int64_t>(nset, geo.nrows - a.s0);
+            a.nspin = L.nspin;
+            a.nb = L.nbnds;
+            a.nspinor = L.nspinor;
+            a.nmag = nmag_eff;
+            a.nzk_max = geo.nzk;
+            a.nst_max = geo.nst;
+            const int64_t planes = (int64_t)a.ns * Nx * a.nv * np;
+            a.sper = (int)std::max<int64_t>(1, std::min<int64_t>(CONV_SETS, planes / 1024));
+            const int64_t blocks = nx8 * a.nv * cdiv(a.ns, a.sper) * np;
+            if (geo.square)
+                LELPH_TRY(conv_square_launch<T>(geo.sqlds, blocks, st, dp, ds, a, Wz));
+            else
+                LELPH_TRY(
+                    conv_plane_launch<T>(geo.two, geo.conv, blocks, st, dp, ds, a, pc, Wy, Wz));
+            const int64_t rows = (int64_t)a.ns * a.nv;
+            a.rows_per_block =
+                (int)std::max<int64_t>(1, std::min<int64_t>(8, rows * tiles * np / 4096));
+            LELPH_TRY(conv_x_launch<T>(geo.xcls, geo.xlds,
+                                       dim3(tiles, (unsigned)cdiv(rows, a.rows_per_block),
+                                            (unsigned)np),
+                                       st, dp, ds, a, Wx));
+        }
+        z64* gm = g + m0 * es; // fewer than all modes: of a single pair
+        LELPH_TRY(sph_gemm_launch<T>(geo.nsplit, np, st, dp, ds, nm, L.nspin, L.nbnds,
+                                     L.nspinor, 1.0 / (double)c->nf,
+                                     geo.nsplit > 1 ? b.part.as<z64>() : gm));
+        if (ev && m0 + nm == L.nmodes) HIP_TRY(hipEventRecord(ev[2], st));
+        if (geo.nsplit > 1)
+            LELPH_TRY(reduce_parts(b.part.as<z64>(), geo.nsplit, nm * es * np,
+                                   1.0 / (double)c->nf, gm, st));
     }
     return LELPH_OK;
 }
@@ -435,6 +453,9 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
 static bool conv_use(const lelph_ctx* c, ConvGeo* g)
 {
     if (c->local_form == LELPH_FORM_BOX || c->conv_off || !conv_geo(c, g)) return false;
+    // one pair's buffers in half of the memory: three boxes' worth where the
+    // sphere fills the box, the box form takes two
+    if (ConvLayout(c, *g, conv_group(c, *g, 1), 1, 2).bytes() > c->mem_total / 2) return false;
     if (c->local_form == LELPH_FORM_SPHERE) return true;
     const lelph_lattice& L = c->lat;
     const int prec = effective_precision(c), nb = L.nbnds;

@@ -206,6 +206,7 @@ struct lelph_ctx
     bool box_defer = false;
     bool conv_off = false; // a sphere that the sphere form does not take was met
     int local_form = LELPH_FORM_AUTO;
+    size_t mem_total = 0; // of the device
     const void* kq_view = nullptr;
     int kq_g0[3] = {0, 0, 0};
 
@@ -1118,6 +1119,8 @@ static int create_impl(const lelph_lattice* L, const lelph_pseudo* P, int precis
     if (precision < LELPH_FP64 || precision > LELPH_BF16X6) return LELPH_ERR_ARG;
     c->precision = precision;
     HIP_TRY(hipGetDevice(&c->device));
+    size_t mem_free = 0;
+    HIP_TRY(hipMemGetInfo(&mem_free, &c->mem_total));
     {
         double* sp = nullptr;
         LELPH_TRY(scratch_ptr(&sp));
@@ -1958,7 +1961,7 @@ struct lelph_multi
     {
         bool on = false;
         ConvGeo geo;
-        ConvGroup gr{1, 1, 1};
+        ConvGroup gr{1, 1, 1, 1};
         ConvBufs bufs;
         std::vector<DBuf> desc;
         std::vector<lelph_pair> pairs;

@@ -11,6 +11,8 @@ just as well.
 Bars: the FP64 form differs from the oracle by rounding of the same sums
 (1e-10, as everywhere); FP32 transforms of N points carry some
 log2(N) * 6e-8 per coefficient, averaged over the sphere (1e-6)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -89,3 +91,41 @@ def test_bands_and_spin(case, nb, fft):
         ctx.close()
     say(f"case: sphere form {case} nb {nb} {fft}: {errs}")
     assert errs["fp64"] < 1e-10 and errs["fp32"] < 1e-6
+
+
+def test_blocks_of_modes():
+    """A pair whose coefficients on the sphere, 24 modes x 256 bands x 46,000
+    plane waves, exceed the 4 GB kept of them: transformed and contracted in
+    two blocks of modes (16 and 8: 2.9 GB beside the boxes, lines and maps, not
+    4.3).  Against the box form, another sum of the same terms (1e-12; the
+    oracle takes minutes), alone and in a batch of two."""
+    free_total = (ctypes.c_size_t * 2)()
+
+    def free():
+        # the HIP runtime that the library is linked to
+        assert lelph.lib().hipMemGetInfo(free_total, ctypes.byref(free_total, 8)) == 0
+        return free_total[0] / 2 ** 30
+
+    s = synth.make_system("blocks", 11, 16.0 * np.eye(3),
+                          [[x, y, z] for x in (0, 0.5) for y in (0, 0.5) for z in (0, 0.5)],
+                          [0] * 8, [3.0], (48, 48, 48), (2, 1, 1), 77.0, 256,
+                          [(np.eye(3), np.zeros(3), 0)], 0, [(0.5, 0.0, 0.0)])
+    assert 16 * s.nmodes * s.nbnds * min(w.npw for w in s.wfcs) > 4 << 30
+    pairs = synth.kq_pairs(s, 0)
+    g = {}
+    ctx = lelph.Context(s, "fp64")
+    try:
+        ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
+        for form in ("box", "sphere"):
+            ctx.set_local_form(form)
+            before = free()
+            g[form] = np.stack([ctx.elph_local(*p) for p in pairs])
+            used = before - free()
+        say(f"case: sphere form in blocks of modes: {used:.2f} GB of buffers")
+        assert used < 5.2
+        assert np.array_equal(ctx.gkq_batch(pairs, non_loc=False, qpt=s.qpts[0]), g["sphere"])
+    finally:
+        ctx.close()
+    err = rel_err(g["sphere"], g["box"])
+    say(f"  npw {[w.npw for w in s.wfcs]}, against the box form {err:.2e}")
+    assert err < 1e-12
