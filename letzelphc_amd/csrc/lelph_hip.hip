@@ -992,7 +992,7 @@ static int run_local_any(lelph_ctx* c, const double* qpt, const lelph_pair& pr, 
 
 // reads and clears the device error word (bit 0: G outside the box or table
 // range, bit 1: symmetry incompatible with the FFT grid, bit 2: rotated
-// index out of range)
+// index out of range, bit 3: a sphere that the sphere form does not take)
 static int read_err(lelph_ctx* c, int* e)
 {
     *e = 0;
@@ -1002,13 +1002,16 @@ static int read_err(lelph_ctx* c, int* e)
     return LELPH_OK;
 }
 
-static int check_err(lelph_ctx* c)
+// local: after a local part, whose caller goes on in the box form at
+// LELPH_CONV_REDO; no other call has set bit 3, and one that failed in
+// between may have left it
+static int check_err(lelph_ctx* c, bool local = false)
 {
     int e = 0;
     LELPH_TRY(read_err(c, &e));
     if (e & 2) return LELPH_ERR_SYM;
     if (e & 7) return LELPH_ERR_RANGE;
-    if (e) return LELPH_CONV_REDO;
+    if (e && local) return LELPH_CONV_REDO;
     return LELPH_OK;
 }
 
@@ -1733,7 +1736,7 @@ static int one_pair(lelph_ctx* c, const double* qpt, int ikq, int ik, int kqsym,
         LELPH_TRY(gkq_device(c, qpt, pr, local, nonloc, c->g.as<z64>(), c->evs.data()));
         HIP_TRY(hipMemcpyAsync(host_g, c->g.p, sizeof(z64) * gsz,
                                hipMemcpyDeviceToHost, c->stream));
-        const int st = check_err(c);
+        const int st = check_err(c, local != 0);
         if (st == LELPH_CONV_REDO)
         {
             c->conv_off = true;
@@ -1831,7 +1834,7 @@ static int conv_batch(lelph_ctx* c, const ConvGeo& geo, const double* qpt, int64
         return st;
     }
     while (landed < ngroups) LELPH_TRY(land(landed++));
-    LELPH_TRY(check_err(c));
+    LELPH_TRY(check_err(c, true));
     return finish_timings(c, ngroups, npairs);
 }
 }
@@ -2485,7 +2488,7 @@ static int multi_create(int ncells, lelph_ctx* const* ctxs, const double* qpts,
     }
     for (lelph_ctx* c : m->ctx)
     {
-        st = check_err(c);
+        st = check_err(c, true);
         if (st == LELPH_CONV_REDO) c->conv_off = true;
         if (st != LELPH_OK) return fail(st);
     }
