@@ -1308,6 +1308,7 @@ int lelph_upload_wfc(lelph_ctx* c, int64_t ik, const double* wfc, const double* 
 {
     if (!c || ik < 0 || ik >= (int64_t)c->wf.size() || !wfc || !gvec || npw < 1)
         return LELPH_ERR_ARG;
+    c->conv_off = false; // the sphere that was not taken may be this one
     DevWfc& w = c->wf[ik];
     if (w.wfc) (void)hipFree(w.wfc);
     if (w.gvec) (void)hipFree(w.gvec);

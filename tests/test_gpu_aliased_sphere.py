@@ -2,7 +2,8 @@
 waves G and G - N b_1 on one box point, with the same coefficients (the box
 form stores one over the other).  Every entry point finds that out on the
 device and repeats the work in the box form: g bit-identical to a context
-pinned to it, and nothing of it reaches calls that have no local part."""
+pinned to it.  New wavefunctions bring the sphere form back, and nothing of it
+reaches calls that have no local part."""
 import copy
 
 import numpy as np
@@ -39,6 +40,61 @@ def context(s, prec, form="auto"):
     ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
     ctx.set_local_form(form)
     return ctx
+
+
+KINDS = {
+    "plain": dict(nbnds=3),
+    "spin2": dict(nbnds=2, nspin=2, nmag=2),
+    "spinor_nmag4": dict(nbnds=2, nspinor=2, nmag=4),
+}
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_repeated_in_the_box_form(kind, prec):
+    clean = synth.tiny(syms="id", **KINDS[kind])
+    s = aliased(clean)
+    pairs = synth.kq_pairs(s, 0)
+    touched = next(p for p in pairs if IK in p[:2])
+    say(f"case: aliased sphere {kind} {prec}")
+    box = context(s, prec, "box")
+    ref = box.gkq_batch(pairs, qpt=s.qpts[0])
+    one = {p: box.gkq(*p, qpt=s.qpts[0]) for p in pairs}
+    box.close()
+    good = context(clean, prec)
+    want = good.gkq_batch(pairs, qpt=s.qpts[0])
+    for call in ("gkq", "batch", "compute", "multi"):
+        ctx = context(s, prec)
+        try:
+            assert ctx.local_form() == "sphere"
+            if call == "gkq":
+                free = next(p for p in pairs if IK not in p[:2])
+                ctx.gkq(*free, qpt=s.qpts[0])
+                assert ctx.local_form() == "sphere"
+                assert np.array_equal(ctx.gkq(*touched, qpt=s.qpts[0]), one[touched])
+            elif call == "batch":
+                assert np.array_equal(ctx.gkq_batch(pairs, qpt=s.qpts[0]), ref)
+            elif call == "compute":
+                assert np.array_equal(ctx.compute_elphq(s.qpts[0]), ref)
+            else:
+                m = lelph.MultiBatch([(good, s.qpts[0], pairs), (ctx, s.qpts[0], pairs)])
+                try:
+                    for _ in range(3):
+                        a, b = m.run()
+                        assert np.array_equal(a, want) and np.array_equal(b, ref)
+                        good.gkq(*touched, qpt=s.qpts[0])
+                finally:
+                    m.close()
+            assert ctx.local_form() == "box" and good.local_form() == "sphere"
+            w = clean.wfcs[IK]
+            ctx.upload_wfc(IK, w.wfc, w.gvec, w.Fk)
+            assert ctx.local_form() == "sphere"
+            # the K splits of the product follow the largest sphere, now the
+            # clean system's again
+            assert np.array_equal(ctx.gkq_batch(pairs, qpt=s.qpts[0]), want)
+        finally:
+            ctx.close()
+    good.close()
 
 
 @pytest.mark.parametrize("call", ["gkq", "batch"])
