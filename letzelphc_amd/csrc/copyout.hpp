@@ -21,6 +21,15 @@
 #define COPY_OUT_SLOTS 16
 #define COPY_OUT_THREADS 8
 
+// whether the host cannot read or write at p, which the copy engine can
+static bool device_only(const void* p)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeDevice;
+    (void)hipGetLastError(); // memory that HIP does not know: the host's
+    return false;
+}
+
 struct CopyOut
 {
     char* ring = nullptr; // COPY_OUT_SLOTS pinned chunks
@@ -55,7 +64,7 @@ struct CopyOut
     {
         const size_t n = (bytes + COPY_OUT_CHUNK - 1) / COPY_OUT_CHUNK;
         const unsigned cpus = std::thread::hardware_concurrency();
-        if (bytes < COPY_OUT_MIN || cpus < 4 || ensure() != LELPH_OK)
+        if (bytes < COPY_OUT_MIN || cpus < 4 || device_only(dst) || ensure() != LELPH_OK)
         {
             HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
             HIP_TRY(hipStreamSynchronize(st));

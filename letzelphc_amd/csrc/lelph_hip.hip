@@ -1316,11 +1316,18 @@ int lelph_upload_wfc(lelph_ctx* c, int64_t ik, const double* wfc, const double* 
     w = DevWfc{};
     const int64_t nset = (int64_t)c->lat.nspin * c->lat.nbnds * c->lat.nspinor;
     w.npw = npw;
+    std::vector<double> gv; // the G list where the host can read it
+    if (device_only(gvec))
+    {
+        gv.resize(3 * (size_t)npw);
+        HIP_TRY(hipMemcpy(gv.data(), gvec, sizeof(double) * gv.size(), hipMemcpyDeviceToHost));
+    }
+    const double* hg = gv.empty() ? gvec : gv.data();
     const double* kp = c->kpt_ibz.data() + 3 * ik;
     for (int64_t g = 0; g < npw; ++g)
     {
-        const double x = kp[0] + gvec[3 * g], y = kp[1] + gvec[3 * g + 1],
-                     z = kp[2] + gvec[3 * g + 2];
+        const double x = kp[0] + hg[3 * g], y = kp[1] + hg[3 * g + 1],
+                     z = kp[2] + hg[3 * g + 2];
         w.rmax = std::max(w.rmax, x * x + y * y + z * z);
     }
     w.rmax = sqrt(w.rmax);
