@@ -41,6 +41,7 @@ struct CopyOut
         if (!ring && hipHostMalloc(reinterpret_cast<void**>(&ring),
                                    COPY_OUT_CHUNK * COPY_OUT_SLOTS) != hipSuccess)
         {
+            (void)hipGetLastError(); // plain copies then; no launch shall report it
             ring = nullptr;
             return LELPH_ERR_ALLOC;
         }
