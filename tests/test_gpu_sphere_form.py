@@ -56,6 +56,35 @@ def test_grids(fft):
     assert errs["fp64"] < 1e-10 and errs["fp32"] < 1e-6
 
 
+# square planes that GRIDS leaves out
+SQUARES = [18, 20, 24, 25, 27, 28, 32, 36, 40, 42, 48, 50, 54, 60, 64, 70, 72, 75, 80, 81, 84, 90,
+           100, 108, 120]
+
+
+@pytest.mark.parametrize("n", SQUARES)
+def test_square_planes(n):
+    s = synth.tiny(nbnds=4, fft=(12, n, n), kgrid=(2, 2, 1), syms="trev", ecut=6.0,
+                   q=(0.5, 0.0, 0.0))
+    o = O.OracleSystem(s)
+    dv = o.dv_total(0)
+    pairs = synth.kq_pairs(s, 0)
+    pick = [pairs[0], pairs[-1]]
+    ref = np.stack([o.elph_local(0, *p, dv) for p in pick])
+    errs = {}
+    ctx = lelph.Context(s, "fp64")
+    try:
+        ctx.set_local_form("sphere")
+        ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
+        for prec in ("fp64", "fp32"):
+            ctx.set_precision(prec)
+            assert ctx.local_form() == "sphere"
+            errs[prec] = rel_err(ctx.gkq_batch(pick, non_loc=False, qpt=s.qpts[0]), ref)
+    finally:
+        ctx.close()
+    say(f"case: square planes {n}: {errs}")
+    assert errs["fp64"] < 1e-10 and errs["fp32"] < 1e-6
+
+
 SPIN = {
     "spin2": dict(nspin=2, nmag=2),
     "spinor_nmag1": dict(nspinor=2, nmag=1),
