@@ -437,6 +437,44 @@ static int conv_local(lelph_ctx* c, const ConvGeo& geo, ConvBufs& b, DBuf& desc,
 // on one box point); the caller goes on in the box form
 #define LELPH_CONV_REDO 1001
 
+// Sticks per (Gy, Gz) of the plane up to which conv_use's constants hold: a
+// sphere of half a grid's length across takes (1/2 + 1/N)^2 of them.
+static const double CONV_ORDINARY = 0.34;
+
+// The same question for spheres that fill more of the box than that.  The
+// sphere form keeps more columns, sticks and plane waves there: at 60^3, 64
+// bands, 18 modes, FP32, a sphere of 0.47, 0.60, 0.76, 0.93 of an axis takes
+// 3.7, 5.2, 7.7, 11.7 ps against the box form's 7.0.  Both forms in ps per
+// pair, fitted to 1900 timings (12^3 to 80^3, slabs, 4 to 128 bands, spheres
+// of 0.47 to 0.93, one to four pairs, all spins; rms 6 to 15 %): launches,
+// psi boxes per row and point, the rest per mode, row and point.  With
+// conv_use's constants alone 160 of them took the sphere form at up to 2.3
+// times the box form's time; 25 do with this, at up to 1.25.
+static bool conv_dense(const lelph_ctx* c, const ConvGeo& g, int prec, double box, double fs)
+{
+    const lelph_lattice& L = c->lat;
+    const double rows = (double)c->nf * L.nspin * L.nspinor * L.nbnds, work = rows * L.nmodes;
+    const double fp = (double)g.npw / (double)c->nf;
+    double tb;
+    if (prec == LELPH_FP64)
+        tb = g.two ? 14 * rows + (box + 3.2) * work : 28 * rows + (box + 1.8) * work;
+    else if (prec == LELPH_FP32)
+        tb = 21 * rows + (g.two ? 1.95 : 1.0) * box * work;
+    else if (prec == LELPH_BF16X6)
+        tb = g.two ? 21 * rows + (1.7 * box + 0.7) * work : 28 * rows + box * work;
+    else
+        tb = 28 * rows + 0.8 * box * work;
+    double ts; // without the sticks' and the product's share
+    if (g.f32)
+        ts = g.two ? 14 * rows + 2.7 * work : (g.square ? 23 : 26) * rows;
+    else
+        ts = g.two ? 54 * rows + 4.5 * work
+                   : g.square ? 28 * rows + 1.2 * work : 45 * rows;
+    const double stick = g.f32 ? (g.two ? 8.3 : g.square ? 7.2 : 9.7)
+                               : (g.two ? 14.8 : g.square ? 12.2 : 17.7);
+    return 40e6 + ts + (stick * fs + 0.18 * fp * L.nbnds) * work < 95e6 + tb;
+}
+
 // Whether the local part runs in the sphere form.  Per set, mode and grid
 // point the box form costs 8 nb operations, the sphere form a transform
 // whatever nb is; measured in picoseconds (60^3 .. 96^3, 16 .. 128 bands,
@@ -459,9 +497,7 @@ static bool conv_use(const lelph_ctx* c, ConvGeo* g)
     if (c->local_form == LELPH_FORM_SPHERE) return true;
     const lelph_lattice& L = c->lat;
     const int prec = effective_precision(c), nb = L.nbnds;
-    // a pair whose box product takes less than some 100 us
     const double work = (double)c->nf * L.nmodes * L.nspin * L.nspinor * nb; // points x rows
-    if (work < 2e7) return true;
     double box, sphere;
     if (prec == LELPH_FP64)
     {
@@ -482,8 +518,10 @@ static bool conv_use(const lelph_ctx* c, ConvGeo* g)
             box = 2.65 * (double)(cdiv(nb, 16) * 16) * (double)(cdiv(nb, 128) * 128) /
                   (128.0 * nb);
     }
-    if (g->two && prec != LELPH_BF16X6) box *= 2.2;
-    return sphere < box;
+    // below 2e7 the box product of a pair takes less than some 100 us
+    if (work >= 2e7 && sphere >= box * (g->two && prec != LELPH_BF16X6 ? 2.2 : 1)) return false;
+    const double fs = (double)g->nst / (double)(L.fft_dims[1] * L.fft_dims[2]);
+    return fs <= CONV_ORDINARY || conv_dense(c, *g, prec, box, fs);
 }
 
 // the potential in the precision that the sphere form reads

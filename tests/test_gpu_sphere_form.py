@@ -158,3 +158,38 @@ def test_blocks_of_modes():
     err = rel_err(g["sphere"], g["box"])
     say(f"  npw {[w.npw for w in s.wfcs]}, against the box form {err:.2e}")
     assert err < 1e-12
+
+
+# (points per axis, bands): where spheres that fill the box make the sphere
+# form the slower one (a sphere of 0.92 of an axis; 1.3 to 1.9 times the box
+# form's time when it was taken there all the same)
+DENSE = [((48, 48, 48), 32, "fp64"), ((48, 48, 48), 64, "fp32"), ((45, 45, 108), 32, "fp64"),
+         ((48, 60, 72), 8, "fp64"), ((48, 60, 72), 64, "bf16x6")]
+
+
+@pytest.mark.parametrize("fft,nb,prec", DENSE)
+def test_spheres_that_fill_the_box(fft, nb, prec):
+    """the box form by itself for a dense sphere, the sphere form for one of
+    half an axis, and both forms of the dense one agree"""
+    used, g = {}, {}
+    for frac in (0.235, 0.46):
+        gmax = frac * 3.0 * 2 * np.pi  # points per bohr: 3
+        s = synth.make_system("dense", 5, np.diag(np.array(fft) / 3.0),
+                              [[0, 0, 0], [0.5, 0.5, 0.5], [0.5, 0.0, 0.5], [0.0, 0.5, 0.5]],
+                              [0] * 4, [3.0], fft, (2, 1, 1), gmax ** 2, nb,
+                              [(np.eye(3), np.zeros(3), 0)], 0, [(0.5, 0.0, 0.0)])
+        ctx = lelph.Context(s, prec)
+        try:
+            used[frac] = ctx.local_form()
+            if frac > 0.4:
+                ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
+                pair = synth.kq_pairs(s, 0)[0]
+                for form in ("auto", "sphere"):
+                    ctx.set_local_form(form)
+                    g[form] = ctx.elph_local(*pair)
+        finally:
+            ctx.close()
+    err = rel_err(g["sphere"], g["auto"])
+    say(f"case: dense sphere {fft} nb {nb} {prec}: {used}, the forms {err:.2e} apart")
+    assert used == {0.235: "sphere", 0.46: "box"}
+    assert err < (1e-12 if prec == "fp64" else 1e-6)
