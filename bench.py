@@ -10,9 +10,11 @@ host.  Metric: g elements/s = pairs * modes * bands^2 / wall time of a step.
 The headline variant (--precision, default: the fastest variant that stays
 within |dg|/|g|max <= 1e-6 of the GPU FP64 result) is timed beside the
 plain FP64 path; both throughputs and their ratio are in the JSON line.
-Roofline: the local contraction kernel, algorithmic 8 flops per complex MAC
-times nmodes*nspin*nb^2*nspinor*N MACs per (k,q) launch, over its mean
-launch time from HIP events on the library stream.
+Roofline: the local part's matrix elements, over their mean time per pair from
+HIP events on the library stream.  Operations as the form that ran needs them:
+contracted over the box, 8 flops per complex MAC times nmodes*nspin*nb^2*
+nspinor*N MACs; transformed to the k+q sphere, per mode and set 6 N for dV psi,
+5 N log2 N for its transform and 8 npw nb for the product.
 """
 from __future__ import annotations
 
@@ -59,6 +61,15 @@ def run_variant(ctx, pairs, prec, steps, warmup):
             f"{tm['contract_ms']:.1f} ms, boxes {tm['boxes_ms']:.1f} ms, "
             f"non-local {tm['nonlocal_ms']:.1f} ms over {tm['pairs']} pairs")
     return out.copy(), np.array(walls), np.array(contract), np.array(total)
+
+
+def local_flops(s, npw, form):
+    """operations of one pair's local part, boxes aside, in the form that ran"""
+    sets = s.nmodes * s.nspin * s.nbnds * s.nspinor
+    n = float(s.nfft)
+    if form == "box":
+        return 8.0 * n * sets * s.nbnds
+    return sets * (6 * n + 5 * n * np.log2(n) + 8.0 * npw * s.nbnds)
 
 
 def cpu_baseline(sys_, pairs, dv, cores):
@@ -404,10 +415,18 @@ def main():
         f"dV set-up {t_dv:.2f} s)")
 
     g64, w64, c64, _ = run_variant(ctx, pairs, "fp64", args.steps, args.warmup)
+    forms = {"fp64": ctx.local_form()}
     variants = ["bf16x6", "bf16x3", "fp32"] if args.precision == "auto" else [args.precision]
-    results = {}
+    results, as_fp32 = {}, []
     head = None
     for v in variants:
+        ctx.set_precision(v)
+        forms[v] = ctx.local_form()
+        if forms[v] == "sphere" and v != "fp32" and "fp32" in variants:
+            # the sphere form knows FP32 and FP64 storage: this run is fp32's
+            as_fp32.append(v)
+            log(f"{v}: runs as fp32 (sphere form), not timed again")
+            continue
         try:
             gv, wv, cv, _ = run_variant(ctx, pairs, v, args.steps, args.warmup)
         except lelph.LelphError as e:
@@ -427,7 +446,8 @@ def main():
     ms = float(np.mean(wv)) * 1e3
     value = nel / (ms / 1e3)
     v64 = nel / float(np.mean(w64))
-    flop_launch = 8.0 * s.nspinor * s.nfft * s.nmodes * s.nspin * s.nbnds ** 2
+    flop_launch = local_flops(s, float(np.mean(npw)), forms[head])
+    flop64_launch = local_flops(s, float(np.mean(npw)), forms["fp64"])
     t_launch = float(np.mean(cv)) / len(pairs) / 1e3
     achieved = flop_launch / t_launch / 1e12
     peak = PEAK_TFLOPS[head]
@@ -482,15 +502,19 @@ def main():
                                f"{len(pairs)} (k,k+q) pairs of q={tuple(float(x) for x in s.qpts[0])}, "
                                f"{s.nmodes} modes, {s.nbnds} bands, npw {min(npw)}..{max(npw)}",
                    "variant": head, "pairs": len(pairs)},
-        "variants": {k: {"g_per_s": nel / float(np.mean(v[0])), "rel_err_vs_fp64": v[2],
+        "variants": {k: {"form": forms[k], "g_per_s": nel / float(np.mean(v[0])), "rel_err_vs_fp64": v[2],
                          "contract_ms_per_pair": float(np.mean(v[1])) / len(pairs)}
                      for k, v in results.items()},
-        "fp64": {"g_per_s": v64, "contract_ms_per_pair": t64_launch * 1e3,
-                 "contract_tflops": flop_launch / t64_launch / 1e12},
+        "runs_as_fp32": as_fp32,
+        "fp64": {"form": forms["fp64"], "g_per_s": v64,
+                 "contract_ms_per_pair": t64_launch * 1e3,
+                 "contract_tflops": flop64_launch / t64_launch / 1e12},
         "ratio_vs_fp64": value / v64,
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
                      "frac": achieved / peak, "traffic": traffic,
-                     "kernel": ({"bf16x3": "k_contract_split_pc", "bf16x6": "k_contract_split"}
+                     "kernel": ("k_conv_square, k_conv_x, k_sph_gemm (transforms of dV psi and "
+                                "the product over the sphere)" if forms[head] == "sphere" else
+                                {"bf16x3": "k_contract_split_pc", "bf16x6": "k_contract_split"}
                                 .get(head, "k_contract")
                                 + f" ({head}, {PRODUCTS[head]} MFMA product(s) per real product; "
                                   "achieved counts the 8 useful flops per complex MAC)"),
@@ -507,7 +531,7 @@ def main():
             "real_space_mflop_per_g": real_mf, "reference_mflop_per_g": ref_mf,
             "reference_equivalent_tflops": value * ref_mf * 1e6 / 1e12,
             "note": "the reference's FFT-convolution + sphere ZGEMM work per g element "
-                    "against this build's real-space contraction"},
+                    "(the sphere form's too) against a real-space contraction"},
         "cpu_baseline": cpu,
         "aux": aux,
     }
