@@ -313,9 +313,7 @@ __device__ __forceinline__ void ln_second(const cpx<T>* row, int k1, cpx<A>* v)
     Rdft<A, SIGN, R2>::run(v);
 }
 
-// exchange row of a line, in elements: of the strides near the least one it
-// has (close to) the fewest bank conflicts of the lanes' two access patterns
-// (96 points: 64 against 96 LDS cycles with an odd one)
+// exchange row of a line, in elements: [R2][R1 | 1]
 constexpr int ln_row(int R1, int R2) { return R2 * (R1 | 1); }
 // the same for the x steps, whose lanes run over lines (odd)
 constexpr int ln_xrow(int R1, int R2) { return (R2 * (R1 | 1)) | 1; }
@@ -694,9 +692,9 @@ constexpr int sq_groups(int R1, int R2, int NW)
 // twiddles in LDS instead of 4 (R1 - 1) registers
 constexpr bool sq_tw_lds(int R1) { return R1 >= 7; }
 // row groups of a plane whose dV stays in registers over the sets: in FP32
-// what fits in 40 of them (a 96 x 96 plane then loads 74 KB and not 147 per
-// set: 22.1 -> 17.3 ms per pair of the 128-band cell, all steps); in FP64
-// none (64 registers of it made the transforms spill: 31.9 -> 34.1 ms)
+// what fits in 40 of them (72^3, 64 bands, 4 pairs: 13.6 -> 13.1 ms; 96^3,
+// 128 bands: no difference, 19.8 ms per pair either way); in FP64 none (64
+// registers of it made the transforms spill: 31.9 -> 34.1 ms per pair)
 template <typename T>
 constexpr int sq_keep(int R1, int R2, int NW)
 {

@@ -4,8 +4,8 @@
 
 #include "conv.hpp"
 
-// threads of a plane block: 512 where the exchange rows and the plane buffer
-// fit in LDS (short factors only), else 256; 0: neither fits.
+// a plane block: class of its line lengths (rx_class), threads (a multiple of
+// 64 up to plane_threads in k_conv_plane, 256 or 512 in k_box_plane) and LDS
 struct PlaneShape
 {
     int cls, nt;

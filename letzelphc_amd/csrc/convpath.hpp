@@ -25,13 +25,14 @@ struct ConvGeo
 
 // bytes of line buffers (the planes' output) that a launch may fill.  More
 // than the 256 MB last-level cache on purpose: fewer, longer launches and
-// more sets per psi plane outweigh what the x step finds cached (96^3, FP64,
-// per pair: 39.7 ms with 128 MB, 35.6 with 512, 34.6 with 1000; a slab's 36
-// pairs 15.1 ms with 512, 14.1 with 1024)
+// more sets per psi plane outweigh what the x step finds cached (4 pairs of
+// 96^3, 128 bands, FP64: 153 ms with 128 MB, 133 with 512, 128 with 1024, 126
+// with 2048; 36 of a 45x45x108 slab 20.2, 14.9, 13.9, 13.6)
 static const int64_t CONV_LINE_BYTES = 1024ll << 20;
-// modes of a launch that share a psi plane in L2 (4: 3 % slower in FP32, 16:
-// no gain), sets that a block takes in turn (32: the blocks of one psi plane
-// drift apart and miss, 3 %; 4: 2 % in starting blocks)
+// modes of a launch that share a psi plane in L2 (96^3 in FP64: 4 costs 5 %,
+// 16 2 %; 72^3 in FP32: 1 % either way), sets that a block takes in turn (96^3:
+// 32 cost 3 %, the blocks of one psi plane drift apart and miss, 4 cost 2 % in
+// starting blocks; 72^3 in FP32: 32 gain 2 to 3 %, 4 cost 8 %)
 static const int CONV_MODES = 8, CONV_SETS = 8;
 static const int64_t CONV_GROUP_BYTES = 2ll << 30;
 // bytes of a pair's coefficients on the k+q sphere, all sets of a block of
@@ -477,17 +478,22 @@ static bool conv_dense(const lelph_ctx* c, const ConvGeo& g, int prec, double bo
 
 // Whether the local part runs in the sphere form.  Per set, mode and grid
 // point the box form costs 8 nb operations, the sphere form a transform
-// whatever nb is; measured in picoseconds (60^3 .. 96^3, 16 .. 128 bands,
-// all steps of the local part):
-//   box, FP32    0.093 per band, bands padded to 16 (57 ms per 96^3 pair of
-//                128 bands and 48 modes); FP64 0.19, with the padding of
-//                its tile; bf16x6 5.4 per tile of 128 x 64; bf16x3 on the
-//                producer/consumer kernel 2.65 at 128 bands
+// whatever nb is; in picoseconds, all steps of the local part:
+//   box, FP32    0.093 per band, bands padded to 16; FP64 0.19, with the
+//                padding of its tile; bf16x6 5.4 per tile of 128 x 64; bf16x3
+//                on the producer/consumer kernel 2.65 at 128 bands
 //   sphere       square planes 3.3 + 0.011 nb (FP32), 5.6 (FP64), others
 //                4.5 + 0.011 nb and 6.0; a 2x2 spinor potential 5.2 and 14
 //                (box form 2.2 x)
-// Where the box form's time is a few launches, the sphere form wins by
-// taking all pairs of a group together.
+// Fitted to the first kernels of the sphere form.  Measured since, 96^3, 128
+// bands, 48 modes, per pair: FP64 29.4 ms (5.4 ps) against 133.5 (24.6) in the
+// box form, FP32 19.9 (3.7) against 58.9 (10.8), bf16x6 31.7 (5.8), bf16x3
+// 16.1 (3.0).  So the rule stays with the box form a little longer than it
+// needs to: in 26 of 322 timings of spheres of half an axis (FP32 at 16 and 32
+// bands on 36^3 to 80^3, FP64 at 16) the sphere form would take 0.5 to 0.97 of
+// the time; it takes none where the box form is more than 2 % faster.
+// Below 2e7 points x rows, where the box form's time is launches, the sphere
+// form wins by taking all pairs of a group together.
 static bool conv_use(const lelph_ctx* c, ConvGeo* g)
 {
     if (c->local_form == LELPH_FORM_BOX || c->conv_off || !conv_geo(c, g)) return false;
@@ -518,7 +524,10 @@ static bool conv_use(const lelph_ctx* c, ConvGeo* g)
             box = 2.65 * (double)(cdiv(nb, 16) * 16) * (double)(cdiv(nb, 128) * 128) /
                   (128.0 * nb);
     }
-    // below 2e7 the box product of a pair takes less than some 100 us
+    // below 2e7 the box product of a pair takes less than some 100 us; all
+    // pairs of a group in one launch each then save more than it costs (64
+    // pairs of 24^3, 8 bands: 6.6 -> 0.6 ms; a single pair, 16 bands: 0.157
+    // against 0.168 ms of local part)
     if (work >= 2e7 && sphere >= box * (g->two && prec != LELPH_BF16X6 ? 2.2 : 1)) return false;
     const double fs = (double)g->nst / (double)(L.fft_dims[1] * L.fft_dims[2]);
     return fs <= CONV_ORDINARY || conv_dense(c, *g, prec, box, fs);

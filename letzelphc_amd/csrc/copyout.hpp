@@ -4,7 +4,7 @@
 // bound by one host thread that faults the pages in and copies: 10 GB/s for
 // 85 MB (64 potentials of a 24^3 cell, 8.3 ms beside 0.2 ms of kernels),
 // against 57 GB/s into pinned memory.  Here the chunks land in a pinned ring
-// and a few threads move them on, so the faults run in parallel: 8.5 -> 5.6
+// and a few threads move them on, so the faults run in parallel: 8.4 -> 5.9
 // ms (chunks of 1 MB 7.8, of 512 KB 10: the threads wake each other too often).
 #pragma once
 

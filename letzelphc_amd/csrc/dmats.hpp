@@ -87,8 +87,8 @@ __device__ inline void dm_su2(const z64* su, z64& u, z64& d)
 // what a D matrix finds cleared: no partner anywhere, zero where a partner is
 // missing, no error.  One launch for what were three fills: a D matrix of a
 // small crystal is bound by its launches (45 x 45 x 108 slab, 40 bands, two D
-// matrices and a rotated g per point: 145 -> 119 us with 5 launches per
-// matrix, not 9).
+// matrices and a rotated g per point, 16 points: 326 -> 267 us each with 5
+// launches per matrix, not 9).
 __global__ void k_dm_clear(int* __restrict__ map, int64_t nf, z64* __restrict__ wS2, int64_t n,
                            int* __restrict__ err)
 {

@@ -199,7 +199,7 @@ struct lelph_ctx
     DBuf box_x;
     const void* box_head = nullptr;
     int box_head_ik = -1, box_head_sym = -1, box_head_prec = -1;
-    int64_t box_sides = 0; // psi sides transformed since the call began
+    int64_t box_sides = 0; // psi boxes formed since the call began
     // k+q box in k-side form, its umklapp phase left to the presplit (set
     // around build_boxes by the bf16 split paths); where build_boxes left
     // the k+q box and the umklapp vector its consumer applies
