@@ -514,6 +514,29 @@ __global__ __launch_bounds__(256) void k_reduce_parts(const z64* __restrict__ pa
 {
     reduce_body(part, nsplit, count, scale, gptr<double>::of(g));
 }
+// the same sums, in the same order, of up to 8 parts: one thread per element,
+// all its loads in flight.  With eight threads each most of them have nothing
+// to load (900 bands, 12 modes, 1 part: 0.05 against 0.14 ms).
+__global__ __launch_bounds__(256) void k_reduce_few(const z64* __restrict__ part, int nsplit,
+                                                    int64_t count, double scale,
+                                                    z64* __restrict__ g)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= count) return;
+    z64 p[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+        if (s < nsplit) p[s] = part[(int64_t)s * count + i];
+    double re = 0, im = 0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+        if (s < nsplit)
+        {
+            re += p[s].x;
+            im += p[s].y;
+        }
+    g[i] = {scale * re, scale * im};
+}
 
 // dst[i] = (float) src[i]
 __global__ void k_z64_to_c32(const z64* __restrict__ s, c32* __restrict__ d, int64_t n)

@@ -811,12 +811,16 @@ static void launch_contract(int shape, bool sep, dim3 grid, hipStream_t st, cons
 
 static int effective_precision(const lelph_ctx* c);
 
-// g = scale * the sum of nsplit partials (k_reduce_parts)
+// g = scale * the sum of nsplit partials
 static int reduce_parts(const z64* part, int nsplit, int64_t count, double scale, z64* g,
                         hipStream_t st)
 {
-    hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(count, RP_ELEMS)), dim3(256), 0, st,
-                       part, nsplit, count, scale, g);
+    if (nsplit <= 8)
+        hipLaunchKernelGGL(k_reduce_few, dim3((unsigned)cdiv(count, 256)), dim3(256), 0, st, part,
+                           nsplit, count, scale, g);
+    else
+        hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(count, RP_ELEMS)), dim3(256), 0, st,
+                           part, nsplit, count, scale, g);
     HIP_TRY(hipGetLastError());
     return LELPH_OK;
 }

@@ -52,3 +52,26 @@ def test_tile_shapes(case, prec):
         assert err < (1e-10 if prec == "fp64" else 1e-6)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("target", [1, 6, 21, 24, 27, 48, 300])
+def test_split_sums(target):
+    """the fixed-order sum of the K splits: 1, 2, 7, 8 and 9 parts (up to 8 by
+    one thread per element, more by eight), 16 and 86.  6 modes, 24 bands: 3
+    blocks of the tile that sets the splits, 256 chunks of the 16^3 grid."""
+    s = synth.tiny(nbnds=24, ecut=14.0, fft=(16, 16, 16))
+    o = O.OracleSystem(s)
+    pair = synth.kq_pairs(s, 0)[1]
+    ref = o.elph_local(0, *pair, o.dv_total(0))
+    ctx = lelph.Context(s, "fp64")
+    try:
+        ctx.set_local_form("box")
+        ctx.set_dvscf(s.qpts[0], s.eigvec(0), s.dvscf(0), kernel="dfpt")
+        ctx.set_tuning(split_target=target)
+        g = ctx.elph_local(*pair)
+        assert np.array_equal(g, ctx.elph_local(*pair))
+    finally:
+        ctx.close()
+    err = rel_err(g, ref)
+    say(f"case: split sums, target {target}: {err:.2e}")
+    assert err < 1e-10
