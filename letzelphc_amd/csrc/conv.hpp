@@ -28,6 +28,8 @@
 // transformed in place (a thread writes back the addresses it read).
 #pragma once
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "mfma.hpp"
 #include "radix.hpp"
@@ -552,6 +554,16 @@ constexpr int ln_row_bytes(int R1, int R2)
 // multiple of R2) write a row of their own that nobody reads
 constexpr int ln_space(int R2) { return ln_rows(R2) + (64 % R2 ? 1 : 0); }
 
+// Bytes from the start of the exchange rows that ln_exchange reads: lanes past
+// the last line (R1 < R2: more of them in the second step) read on beyond the
+// rows of their wave, values that are not stored.  A block has at least that
+// much LDS; only planes of a few kept columns have less by themselves.
+static inline size_t ln_reach(int R1, int R2, int NW, int row_bytes)
+{
+    const size_t last = (size_t)(63 / R1) * ln_row(R1, R2) + (R2 - 1) * (R1 | 1) + R1; // of 8 bytes
+    return (size_t)(NW - 1) * ln_space(R2) * row_bytes + 8 * last;
+}
+
 // The exchange of a wave's lines between their two steps: x (twiddled) of
 // lane (row r, j) to v of lane (row rd, k1).  All lanes take part, so there
 // is no branch to carry registers over: rows past LR hold or read values
@@ -754,8 +766,20 @@ static inline PlaneLds plane_lds(int R1y, int R2y, int R1z, int R2z, int nzk, in
     l.tw = (int)(((size_t)l.rows + sizeof(cpx<T>) * (size_t)nzk * l.prow +
                   2 * (size_t)(R1y * R2y + R1z * R2z + nzk * R1y * R2y) + 15) &
                  ~(size_t)15);
-    l.bytes = (size_t)l.tw + sizeof(cpx<T>) * (size_t)(R1y * R2y + R1z * R2z);
+    l.bytes = std::max((size_t)l.tw + sizeof(cpx<T>) * (size_t)(R1y * R2y + R1z * R2z),
+                       ln_reach(R1z, R2z, NT / 64, ln_row_bytes<T>(R1z, R2z)));
     return l;
+}
+
+// the same of k_conv_square: exchange rows, plane buffer, sticks, twiddles
+template <typename T>
+static inline size_t square_lds(int R1, int R2, int NW, int nzk)
+{
+    auto up = [](size_t n) { return (n + 15) & ~(size_t)15; };
+    const size_t rb = (size_t)ln_row_bytes<T>(R1, R2), item = sizeof(cpx<T>);
+    return std::max(up(NW * ln_space(R2) * rb) + up(item * nzk * ln_prow(R1, R2)) +
+                        up(2 * (size_t)nzk * R1 * R2) + (sq_tw_lds(R1) ? item * R1 * R2 : 0),
+                    ln_reach(R1, R2, NW, (int)rb));
 }
 
 // tables of a plane block: address of y inside a column, column of Gz

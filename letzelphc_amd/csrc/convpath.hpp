@@ -118,12 +118,8 @@ static bool conv_geo(const lelph_ctx* c, ConvGeo* g)
     if (g->square)
     {
         const int r1 = g->r1[1], r2 = g->r2[1];
-        const int nw = g->f32 ? rx_square_waves<float>(r1 * r2) : rx_square_waves<double>(r1 * r2);
-        const int rb = g->f32 ? ln_row_bytes<float>(r1, r2) : ln_row_bytes<double>(r1, r2);
-        g->sqlds = (((size_t)nw * ln_space(r2) * rb + 15) & ~(size_t)15) +
-                   ((item * (size_t)g->nzk * ln_prow(r1, r2) + 15) & ~(size_t)15) +
-                   ((2 * (size_t)g->nzk * r1 * r2 + 15) & ~(size_t)15) +
-                   (sq_tw_lds(r1) ? item * r1 * r2 : 0);
+        g->sqlds = g->f32 ? square_lds<float>(r1, r2, rx_square_waves<float>(r1 * r2), g->nzk)
+                          : square_lds<double>(r1, r2, rx_square_waves<double>(r1 * r2), g->nzk);
         g->square = g->sqlds <= 160 * 1024;
     }
     if (!conv_plane_shape(*g, item, cls == 0 ? 512 : 256, false, &g->box)) return false;
